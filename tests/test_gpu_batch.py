@@ -1,0 +1,107 @@
+"""The batched forward at f32 precision (from 84 M weights x batch rows, 56 M
+for Q6_K and Q8_0, on the row-interleaved layouts) at the edges of its tiles,
+with rows of mixed magnitude and non-finite x. Reference: the oracle's f64
+product over the dequantized weights."""
+import numpy as np
+import pytest
+
+import oracle
+import welvet_amd as wv
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5  # the f32 bar of wv_matvec, max |dy| / max |y| of each batch row
+FMTS = ["Q2_K", "Q3_K", "Q4_K", "Q5_K", "Q6_K", "Q8_0", "Q4_0", "Q4_1", "Q5_0", "Q5_1", "IQ1_S", "IQ2_XXS", "IQ2_XS",
+        "IQ3_XXS", "IQ3_S", "IQ4_XS", "IQ4_NL", "TernaryPacked", "BinaryPacked", "AffinePacked"]
+
+
+@pytest.fixture(scope="module", autouse=True)
+def device():
+    print(f"[gpu] {__name__}: init device 0", flush=True)
+    wv.init(0)
+    yield
+
+
+def make(fmt, rows, cols, seed):
+    rng = np.random.default_rng(seed)
+    p = wv.pack(fmt, (rng.standard_normal(rows * cols) * 0.02).astype(np.float32), rows, cols)
+    return p, wv.upload(p), rng
+
+
+def reference(p, x):
+    return oracle.reference_y(oracle.Packed(p.fmt, p.rows, p.cols, p.raw, p.scales, p.meta, p.block_weights, p.mins), x)
+
+
+def rowwise(y, ref):
+    ref = np.asarray(ref, np.float64)
+    return float((np.abs(y - ref).max(1) / np.abs(ref).max(1)).max())
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+def test_batched_forward_formats(fmt):
+    rows, cols = 2000, 2304  # a ragged last row group; 9 super-blocks: waves of two, the last of one
+    print(f"[gpu] batched {fmt}", flush=True)
+    p, d, rng = make(fmt, rows, cols, 11)
+    x = rng.standard_normal((19, cols)).astype(np.float32)  # a block of 16 and one of 3
+    assert rowwise(d.matvec(x), reference(p, x)) <= TOL
+    d.free()
+
+
+@pytest.mark.parametrize("fmt", ["Q4_K", "Q8_0"])
+@pytest.mark.parametrize("shape", [(40001, 256, 9), (14337, 4096, 2), (4099, 4096, 7), (4099, 4096, 8), (4099, 4096, 9),
+                                   (4099, 4096, 16), (2049, 4096, 33), (520, 14336, 17), (65, 14336, 96)])
+def test_batched_forward_tiles(fmt, shape):
+    """One super-block; one row past a row group; batches around the 8 and 16 rows of a block; K split over
+    blocks, down to 4 super-blocks each."""
+    rows, cols, batch = shape
+    print(f"[gpu] batched {fmt} {rows}x{cols} batch {batch}", flush=True)
+    p, d, rng = make(fmt, rows, cols, rows + batch)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    assert rowwise(d.matvec(x), reference(p, x)) <= TOL
+    d.free()
+
+
+@pytest.mark.parametrize("fmt", ["Q4_K", "Q6_K", "Q4_1"])
+def test_batched_forward_magnitudes(fmt):
+    """Each batch row and super-block has its own power of two: rows of 1e-30 and 1e30 beside ordinary
+    ones, an outlier channel (the other columns keep 2^-40 of it), an all-zero row."""
+    rows, cols = 4100, 4096
+    print(f"[gpu] batched magnitudes {fmt}", flush=True)
+    p, d, rng = make(fmt, rows, cols, 3)
+    x = rng.standard_normal((6, cols)).astype(np.float32)
+    x[1] *= np.float32(1e-30)
+    x[2] *= np.float32(1e30)
+    x[3, 77] = 1e6
+    x[4] = 0
+    y, ref = d.matvec(x), reference(p, x)
+    live = [0, 1, 2, 3, 5]
+    assert rowwise(y[live].astype(np.float64), ref[live]) <= TOL
+    assert (y[4] == 0).all()
+    d.free()
+
+
+@pytest.mark.parametrize("fmt", ["Q4_K", "Q6_K", "Q8_0", "Q4_1", "IQ1_S"])
+def test_batched_forward_nonfinite(fmt):
+    """NaN and infinities reach every output of their own row and no other's."""
+    rows, cols = 4100, 4096
+    print(f"[gpu] batched non-finite {fmt}", flush=True)
+    p, d, rng = make(fmt, rows, cols, 4)
+    x = rng.standard_normal((6, cols)).astype(np.float32)
+    ref = reference(p, x)
+    x[1, 3], x[2, 300], x[3, 4095] = np.nan, np.inf, -np.inf
+    y = d.matvec(x)
+    assert np.isnan(y[1]).all() and not np.isfinite(y[2]).any() and not np.isfinite(y[3]).any()
+    live = [0, 4, 5]
+    assert rowwise(y[live].astype(np.float64), ref[live]) <= TOL
+    d.free()
+
+
+def test_batched_forward_route_keeps_the_result():
+    """The same rows below and above the work at which the batched kernel takes over agree to the f32 bar."""
+    rows, cols = 4099, 4096
+    print("[gpu] batched route", flush=True)
+    p, d, rng = make("Q4_K", rows, cols, 6)
+    x = rng.standard_normal((8, cols)).astype(np.float32)
+    y8, y2 = d.matvec(x), np.concatenate([d.matvec(x[i:i + 2]) for i in range(0, 8, 2)])
+    assert rowwise(y8.astype(np.float64), y2) <= TOL
+    d.free()

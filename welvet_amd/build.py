@@ -29,7 +29,7 @@ HIP_FLAGS = [
 ]
 CXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-pthread", "-ffp-contract=off", "-Wall"]
 
-HIP_SOURCES = ["runtime.hip", "gemv.hip", "gemv_rpl.hip", "gemm_rpl.hip", "decode.hip", "native.hip"]
+HIP_SOURCES = ["runtime.hip", "gemv.hip", "gemv_rpl.hip", "gemv_batch.hip", "gemm_rpl.hip", "decode.hip", "native.hip"]
 CXX_SOURCES = ["pack.cpp"]
 
 

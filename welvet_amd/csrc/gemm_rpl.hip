@@ -34,367 +34,16 @@
 
 #include <algorithm>
 #include <cstdint>
-#include <type_traits>
 
+#include "rpl_operands.h"
 #include "wave_ops.h"
 #include "wv_internal.h"
 
 namespace wv {
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-
 constexpr int BK = 64;        // columns per K-step
 constexpr int LDK = BK + 8;   // LDS row stride in halves (144 B: conflict-free 16 B row reads)
-
-__device__ __forceinline__ uint4 ld_nt(const uint4* p) {
-    const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
-    return make_uint4(v.x, v.y, v.z, v.w);
-}
-
-__device__ __forceinline__ uint32_t pack_h2(float a, float b) {
-    const half2v h = {_Float16(a), _Float16(b)};
-    return __builtin_bit_cast(uint32_t, h);
-}
-
-// 8 weights from two spread words (byte b of `se` / `so` = the code of
-// column 2b / 2b + 1 of an 8-column run) -> 4 half2 w = fma(q, sc, mn) in
-// fp16, in k order [0,2,4,6,1,3,5,7].
-// Codes of up to 4 bits convert with v_cvt_scalef32_pk_f16_fp8: a byte q <
-// 16 read as fp8 e4m3 is q * 2^-9 exactly (exponent fields 0 and 1 share the
-// step 2^-9), and the instruction applies the exponent of its f32 scale, so
-// scale 512 gives q as fp16 for two bytes in one instruction. Wider codes
-// (up to 5 bits) take the exponent-byte form: 0x64 | q is 1024 + q in fp16.
-template <int FB>
-__device__ __forceinline__ uint4 dequant8s(uint32_t se, uint32_t so, half2v sc, half2v mn) {
-    half2v q[4];
-    if constexpr (FB <= 4) {
-        q[0] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(se, 512.0f, false);
-        q[1] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(se, 512.0f, true);
-        q[2] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(so, 512.0f, false);
-        q[3] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(so, 512.0f, true);
-    } else {
-        const half2v k1024 = {_Float16(1024.0f), _Float16(1024.0f)};
-        const uint32_t e = 0x64646464u;
-        q[0] = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(e, se, 0x04010400u)) - k1024;
-        q[1] = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(e, se, 0x04030402u)) - k1024;
-        q[2] = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(e, so, 0x04010400u)) - k1024;
-        q[3] = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(e, so, 0x04030402u)) - k1024;
-    }
-    uint32_t p[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) p[i] = __builtin_bit_cast(uint32_t, q[i] * sc + mn);
-    return make_uint4(p[0], p[1], p[2], p[3]);
-}
-
-// Code planes of one 32-column chunk of a k-quant row (lane = row) and, after
-// the lane swaps, the spread words of the MFMA B operands: for 32-row tile T
-// and k16 step kk, lanes 0-31 take columns 16kk + 0..7 of rows 32T + lane and
-// lanes 32-63 columns 16kk + 8..15 of the same rows. FB = code bits (2, 3, 4,
-// 5); the planes are those of the forward kernels (Q4_K nibbles; Q5_K fifth
-// bits; Q2_K / Q3_K two-bit plane and third bits).
-template <int FB>
-struct GemmCodes {
-    struct C { uint4 c; uint32_t h; };
-    static __device__ __forceinline__ C load(const RplArgs& a, int64_t ci, int lane) {
-        C r;
-        if constexpr (FB >= 4) {
-            r.c = ld_nt(reinterpret_cast<const uint4*>(a.codes) + ci * 64 + lane);
-        } else {
-            const uint2 v = reinterpret_cast<const uint2*>(a.codes)[ci * 64 + lane];
-            r.c = make_uint4(v.x, v.y, 0u, 0u);
-        }
-        r.h = (FB == 5 || FB == 3) ? reinterpret_cast<const uint32_t*>(a.hi)[ci * 64 + lane] : 0u;
-        return r;
-    }
-    // se/so[T][kk]: even / odd columns of the lane's 8-column run
-    static __device__ __forceinline__ void spread(const C& c, int lane, uint32_t (&se)[2][2], uint32_t (&so)[2][2]) {
-        const int up = lane >> 5;
-        if constexpr (FB >= 4) {
-            const auto k0 = __builtin_amdgcn_permlane32_swap(c.c.x, c.c.y, false, false);  // columns 0-15
-            const auto k1 = __builtin_amdgcn_permlane32_swap(c.c.z, c.c.w, false, false);  // columns 16-31
-#pragma unroll
-            for (int T = 0; T < 2; ++T) {
-                se[T][0] = k0[T] & 0x0F0F0F0Fu;
-                so[T][0] = (k0[T] >> 4) & 0x0F0F0F0Fu;
-                se[T][1] = k1[T] & 0x0F0F0F0Fu;
-                so[T][1] = (k1[T] >> 4) & 0x0F0F0F0Fu;
-            }
-        } else {  // dword kk holds spread words 4kk..4kk+3; this lane's are 4kk + 2up (+1)
-            const auto p0 = __builtin_amdgcn_permlane32_swap(c.c.x, c.c.x, false, false);
-            const auto p1 = __builtin_amdgcn_permlane32_swap(c.c.y, c.c.y, false, false);
-            const int sh = 4 * up;
-#pragma unroll
-            for (int T = 0; T < 2; ++T) {
-                se[T][0] = (p0[T] >> sh) & 0x03030303u;
-                so[T][0] = (p0[T] >> (sh + 2)) & 0x03030303u;
-                se[T][1] = (p1[T] >> sh) & 0x03030303u;
-                so[T][1] = (p1[T] >> (sh + 2)) & 0x03030303u;
-            }
-        }
-        if constexpr (FB == 5 || FB == 3) {  // top bit of spread word s at bit s of each byte
-            constexpr int top = FB == 5 ? 4 : 2;
-            const auto hh = __builtin_amdgcn_permlane32_swap(c.h, c.h, false, false);
-#pragma unroll
-            for (int T = 0; T < 2; ++T)
-#pragma unroll
-                for (int kk = 0; kk < 2; ++kk) {
-                    const int sb = 4 * kk + 2 * up;
-                    se[T][kk] |= ((hh[T] >> sb) & 0x01010101u) << top;
-                    so[T][kk] |= ((hh[T] >> (sb + 1)) & 0x01010101u) << top;
-                }
-        }
-    }
-};
-
-// Per-format B-operand builders of the GEMM kernels. Ch holds one 32-column
-// chunk of the lane's row (codes, the chunk's metadata, the super-block's
-// scales); bops() returns the fp16 B operands bf[T][kk] of 32-row tile T and
-// k16 step kk, in X's k order [0,2,4,6,1,3,5,7], with the tile row's scales
-// and mins multiplied by its power-of-two row factor wk[T] (RplArgs::wrow)
-// before their fp16 cast.
-template <int FB>
-struct GemmKQ {  // Q2_K, Q3_K, Q4_K, Q5_K: w = (d/255)*u*q + (dmin/127)*m
-    struct Ch { typename GemmCodes<FB>::C c; uint32_t mw; float2 dd; };
-    static __device__ __forceinline__ Ch load(const RplArgs& a, int64_t ci, int64_t si, int j, int lane) {
-        return {GemmCodes<FB>::load(a, ci, lane), reinterpret_cast<const uint32_t*>(a.meta)[(si * 64 + lane) * 8 + j],
-                reinterpret_cast<const float2*>(a.dd)[si * 64 + lane]};
-    }
-    // The lane forms the fp16 scales and mins of its own row (row `lane` of
-    // the group: tile lane / 32) and the lane swap hands each lane both tiles'
-    // pairs, the same values the other lane computed.
-    static __device__ __forceinline__ void bops(const Ch& c, int lane, const float (&wk)[2], half8 (&bf)[2][2]) {
-        float w0 = wk[0], w1 = wk[1];
-        asm("" : "+v"(w0), "+v"(w1));  // a select of values, not an indexed load of the array
-        const float wo = (lane & 32) ? w1 : w0;  // the own row's factor
-        const float d255 = c.dd.x * (wo * (1.0f / 255.0f)), dm127 = c.dd.y * (wo * (1.0f / 127.0f));
-        const uint32_t gm = c.mw;
-        const half2v scp = {_Float16(d255 * float(gm & 0xFFu)), _Float16(d255 * float((gm >> 8) & 0xFFu))};
-        const half2v mnp = {_Float16(dm127 * float(int8_t(gm >> 16))), _Float16(dm127 * float(int32_t(gm) >> 24))};
-        const auto sc2 = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, scp),
-                                                          __builtin_bit_cast(uint32_t, scp), false, false);
-        const auto mn2 = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, mnp),
-                                                          __builtin_bit_cast(uint32_t, mnp), false, false);
-        uint32_t se[2][2], so[2][2];
-        GemmCodes<FB>::spread(c.c, lane, se, so);
-#pragma unroll
-        for (int T = 0; T < 2; ++T) {
-            const half2v sp = __builtin_bit_cast(half2v, uint32_t(sc2[T])), np = __builtin_bit_cast(half2v, uint32_t(mn2[T]));
-            const half2v s0 = {sp.x, sp.x}, s1 = {sp.y, sp.y}, n0 = {np.x, np.x}, n1 = {np.y, np.y};
-            bf[T][0] = __builtin_bit_cast(half8, dequant8s<FB>(se[T][0], so[T][0], s0, n0));
-            bf[T][1] = __builtin_bit_cast(half8, dequant8s<FB>(se[T][1], so[T][1], s1, n1));
-        }
-    }
-};
-
-struct GemmQ6 {  // Q6_K: q = lo4 | hi2 << 4, w = (d/255)*u*(q - 32)
-    struct Ch { uint4 c; uint2 h; uint32_t mw; float d; };
-    static __device__ __forceinline__ Ch load(const RplArgs& a, int64_t ci, int64_t si, int j, int lane) {
-        const uint32_t m = reinterpret_cast<const uint32_t*>(a.meta)[(si * 64 + lane) * 4 + (j >> 1)];
-        return {ld_nt(reinterpret_cast<const uint4*>(a.codes) + ci * 64 + lane),
-                reinterpret_cast<const uint2*>(a.hi)[ci * 64 + lane], m >> (16 * (j & 1)),
-                reinterpret_cast<const float*>(a.dd)[(si * 64 + lane) * 2]};
-    }
-    static __device__ __forceinline__ void bops(const Ch& c, int lane, const float (&wk)[2], half8 (&bf)[2][2]) {
-        typename GemmCodes<4>::C nib{c.c, 0u};
-        uint32_t se[2][2], so[2][2];
-        GemmCodes<4>::spread(nib, lane, se, so);
-        // high-bit dword kk holds spread words 4kk..4kk+3 at bits 2f; this lane's are 4kk + 2up (+1)
-        const int sh = 4 * (lane >> 5);
-        const auto h0 = __builtin_amdgcn_permlane32_swap(c.h.x, c.h.x, false, false);
-        const auto h1 = __builtin_amdgcn_permlane32_swap(c.h.y, c.h.y, false, false);
-        const auto dt = __builtin_amdgcn_permlane32_swap(__float_as_uint(c.d), __float_as_uint(c.d), false, false);
-        const auto mt = __builtin_amdgcn_permlane32_swap(c.mw, c.mw, false, false);
-#pragma unroll
-        for (int T = 0; T < 2; ++T) {
-            se[T][0] |= ((h0[T] >> sh) & 0x03030303u) << 4;
-            so[T][0] |= ((h0[T] >> (sh + 2)) & 0x03030303u) << 4;
-            se[T][1] |= ((h1[T] >> sh) & 0x03030303u) << 4;
-            so[T][1] |= ((h1[T] >> (sh + 2)) & 0x03030303u) << 4;
-            const float d255 = __uint_as_float(dt[T]) * (wk[T] * (1.0f / 255.0f));
-            const _Float16 sc0 = _Float16(d255 * float(mt[T] & 0xFFu)), sc1 = _Float16(d255 * float((mt[T] >> 8) & 0xFFu));
-            const _Float16 mn0 = _Float16(-32.0f) * sc0, mn1 = _Float16(-32.0f) * sc1;
-            const half2v s0 = {sc0, sc0}, s1 = {sc1, sc1}, n0 = {mn0, mn0}, n1 = {mn1, mn1};
-            bf[T][0] = __builtin_bit_cast(half8, dequant8s<6>(se[T][0], so[T][0], s0, n0));
-            bf[T][1] = __builtin_bit_cast(half8, dequant8s<6>(se[T][1], so[T][1], s1, n1));
-        }
-    }
-};
-
-struct GemmQ8 {  // Q8_0: w = scale*q, q int8, 32 bytes per chunk (consecutive columns)
-    struct Ch { uint4 c0, c1; uint32_t sc; };
-    static __device__ __forceinline__ Ch load(const RplArgs& a, int64_t ci, int64_t si, int j, int lane) {
-        const uint4* p = reinterpret_cast<const uint4*>(a.codes) + (ci * 64 + lane) * 2;
-        return {ld_nt(p), ld_nt(p + 1), reinterpret_cast<const uint32_t*>(a.meta)[(si * 64 + lane) * 8 + j]};
-    }
-    static __device__ __forceinline__ void bops(const Ch& c, int lane, const float (&wk)[2], half8 (&bf)[2][2]) {
-        (void)lane;
-        const uint32_t dw[8] = {c.c0.x, c.c0.y, c.c0.z, c.c0.w, c.c1.x, c.c1.y, c.c1.z, c.c1.w};
-        const auto st = __builtin_amdgcn_permlane32_swap(c.sc, c.sc, false, false);
-        const half2v k1152 = {_Float16(1152.0f), _Float16(1152.0f)};
-        const uint32_t e = 0x64646464u;
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            // lanes 0-31: columns 16kk + 0..7 (dwords 4kk, 4kk+1); lanes 32-63: + 8..15
-            const auto A = __builtin_amdgcn_permlane32_swap(dw[4 * kk], dw[4 * kk + 2], false, false);
-            const auto B = __builtin_amdgcn_permlane32_swap(dw[4 * kk + 1], dw[4 * kk + 3], false, false);
-#pragma unroll
-            for (int T = 0; T < 2; ++T) {
-                const uint32_t lo = A[T] ^ 0x80808080u, hi = B[T] ^ 0x80808080u;  // q + 128 as unsigned bytes
-                const uint32_t hb[4] = {__builtin_amdgcn_perm(e, lo, 0x04020400u), __builtin_amdgcn_perm(e, hi, 0x04020400u),
-                                        __builtin_amdgcn_perm(e, lo, 0x04030401u), __builtin_amdgcn_perm(e, hi, 0x04030401u)};
-                const _Float16 sh = _Float16(__uint_as_float(st[T]) * wk[T]);
-                const half2v s2 = {sh, sh};
-                uint32_t p[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) p[i] = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(half2v, hb[i]) - k1152) * s2);
-                bf[T][kk] = __builtin_bit_cast(half8, make_uint4(p[0], p[1], p[2], p[3]));
-            }
-        }
-    }
-};
-
-// The 32-weight block formats (Q4_0 with its nibble xor 8, Q4_1, Q5_0, Q5_1)
-// and AffinePacked g64 (GSH = 1: chunks 2g, 2g+1 share group g): one scale
-// (and min) per chunk from the lane's 8 (16) metadata words per super-block;
-// w = scale*q + min, or scale*(q - OFF).
-template <int FB, bool MIN, int OFF, uint32_t XR, int GSH = 0>
-struct GemmB32 {
-    static constexpr int NG = 8 >> GSH, NW = MIN ? 2 * NG : NG;
-    struct Ch { typename GemmCodes<FB>::C c; uint32_t sc, mn; };
-    static __device__ __forceinline__ Ch load(const RplArgs& a, int64_t ci, int64_t si, int j, int lane) {
-        Ch r;
-        r.c = GemmCodes<FB>::load(a, ci, lane);
-        r.c.c.x ^= XR;
-        r.c.c.y ^= XR;
-        r.c.c.z ^= XR;
-        r.c.c.w ^= XR;
-        const uint32_t* m = reinterpret_cast<const uint32_t*>(a.meta) + (si * 64 + lane) * NW;
-        r.sc = m[j >> GSH];
-        r.mn = MIN ? m[NG + (j >> GSH)] : 0u;
-        return r;
-    }
-    static __device__ __forceinline__ void bops(const Ch& c, int lane, const float (&wk)[2], half8 (&bf)[2][2]) {
-        uint32_t se[2][2], so[2][2];
-        GemmCodes<FB>::spread(c.c, lane, se, so);
-        const auto st = __builtin_amdgcn_permlane32_swap(c.sc, c.sc, false, false);
-        const auto mt = __builtin_amdgcn_permlane32_swap(c.mn, c.mn, false, false);
-#pragma unroll
-        for (int T = 0; T < 2; ++T) {
-            const float scf = __uint_as_float(st[T]) * wk[T];
-            const _Float16 sc = _Float16(scf), mn = _Float16(MIN ? __uint_as_float(mt[T]) * wk[T] : -float(OFF) * scf);
-            const half2v s2 = {sc, sc}, n2 = {mn, mn};
-            bf[T][0] = __builtin_bit_cast(half8, dequant8s<FB>(se[T][0], so[T][0], s2, n2));
-            bf[T][1] = __builtin_bit_cast(half8, dequant8s<FB>(se[T][1], so[T][1], s2, n2));
-        }
-    }
-};
-
-// Codes of one bit (BinaryPacked g32, IQ1_S): one word per chunk whose byte b
-// holds at bit s the code of column 8(s/2) + 2b + s%2.
-struct GemmCodes1 {
-    struct C { uint32_t c; };
-    static __device__ __forceinline__ C load(const RplArgs& a, int64_t ci, int lane) {
-        return {reinterpret_cast<const uint32_t*>(a.codes)[ci * 64 + lane]};
-    }
-    static __device__ __forceinline__ void spread(const C& c, int lane, uint32_t (&se)[2][2], uint32_t (&so)[2][2]) {
-        const auto hh = __builtin_amdgcn_permlane32_swap(c.c, c.c, false, false);
-        const int up = lane >> 5;
-#pragma unroll
-        for (int T = 0; T < 2; ++T)
-#pragma unroll
-            for (int kk = 0; kk < 2; ++kk) {
-                const int sb = 4 * kk + 2 * up;
-                se[T][kk] = (hh[T] >> sb) & 0x01010101u;
-                so[T][kk] = (hh[T] >> (sb + 1)) & 0x01010101u;
-            }
-    }
-};
-
-// The linear-code formats (the linear IQ formats, TernaryPacked, BinaryPacked
-// g32 and g128): w = scale*(q - MID2/2), one scale per 32 columns, two (SG16,
-// one per k16 step) or one per 2^GSH chunks; one-bit codes read +-scale =
-// (2*scale)*(q - 1/2).
-template <int FB, bool SG16, int MID2, int GSH = 0>
-struct GemmLin {
-    using Codes = std::conditional_t<FB == 1, GemmCodes1, GemmCodes<FB>>;
-    static constexpr int NW = SG16 ? 16 : (8 >> GSH);  // metadata words per lane and super-block
-    struct Ch { typename Codes::C c; uint32_t s0, s1; };
-    static __device__ __forceinline__ Ch load(const RplArgs& a, int64_t ci, int64_t si, int j, int lane) {
-        const uint32_t* m = reinterpret_cast<const uint32_t*>(a.meta) + (si * 64 + lane) * NW;
-        const uint32_t s0 = m[SG16 ? 2 * j : (j >> GSH)];
-        return {Codes::load(a, ci, lane), s0, SG16 ? m[2 * j + 1] : s0};
-    }
-    static __device__ __forceinline__ void bops(const Ch& c, int lane, const float (&wk)[2], half8 (&bf)[2][2]) {
-        uint32_t se[2][2], so[2][2];
-        Codes::spread(c.c, lane, se, so);
-        const auto t0 = __builtin_amdgcn_permlane32_swap(c.s0, c.s0, false, false);
-        const auto t1 = __builtin_amdgcn_permlane32_swap(c.s1, c.s1, false, false);
-        constexpr float mul = FB == 1 ? 2.0f : 1.0f, mid = 0.5f * MID2;
-#pragma unroll
-        for (int T = 0; T < 2; ++T)
-#pragma unroll
-            for (int kk = 0; kk < 2; ++kk) {
-                const float scf = __uint_as_float(kk ? t1[T] : t0[T]) * (mul * wk[T]);
-                const _Float16 sc = _Float16(scf), mn = _Float16(-mid * scf);
-                const half2v s2 = {sc, sc}, n2 = {mn, mn};
-                bf[T][kk] = __builtin_bit_cast(half8, dequant8s<FB>(se[T][kk], so[T][kk], s2, n2));
-            }
-    }
-};
-
-// IQ4_NL (quant/iq.go:169-180): w = scale * grid[q], the 16-value float grid
-// (kIQ4NLGrid) as fp16, one scale per 32-column chunk. The codes are Q4_K's
-// nibble planes; the grid is looked up four codes at a time with
-// v_perm_b32 from byte tables of the fp16 values' low and high bytes (codes
-// 0-7 from the first two dwords of a table, 8-15 from the last two, picked
-// per byte by the code's bit 3), and the low and high bytes are interleaved
-// into half2 pairs in k order [0,2,4,6,1,3,5,7].
-struct GemmNL {
-    static constexpr uint16_t h16(int q) { return __builtin_bit_cast(uint16_t, _Float16(kIQ4NLGrid[q])); }
-    static constexpr uint32_t tab(int n, int sh) {  // bytes 4n..4n+3 of the low (sh 0) or high (sh 8) table
-        return uint32_t((h16(4 * n) >> sh) & 0xFF) | uint32_t((h16(4 * n + 1) >> sh) & 0xFF) << 8 |
-               uint32_t((h16(4 * n + 2) >> sh) & 0xFF) << 16 | uint32_t((h16(4 * n + 3) >> sh) & 0xFF) << 24;
-    }
-    struct Ch { GemmCodes<4>::C c; uint32_t s0; };
-    static __device__ __forceinline__ Ch load(const RplArgs& a, int64_t ci, int64_t si, int j, int lane) {
-        return {GemmCodes<4>::load(a, ci, lane), reinterpret_cast<const uint32_t*>(a.meta)[(si * 64 + lane) * 8 + j]};
-    }
-    // fp16 grid values of the 4 codes in the bytes of c: half2 of bytes 0, 1 and of bytes 2, 3
-    static __device__ __forceinline__ void look4(uint32_t c, half2v& q01, half2v& q23) {
-        constexpr uint32_t L0 = tab(0, 0), L1 = tab(1, 0), L2 = tab(2, 0), L3 = tab(3, 0);
-        constexpr uint32_t H0 = tab(0, 8), H1 = tab(1, 8), H2 = tab(2, 8), H3 = tab(3, 8);
-        const uint32_t sel = c & 0x07070707u;
-        const uint32_t hi8 = ((c >> 3) & 0x01010101u) * 0xFFu;  // 0xFF in the bytes of codes 8-15
-        const uint32_t lo = (__builtin_amdgcn_perm(L3, L2, sel) & hi8) | (__builtin_amdgcn_perm(L1, L0, sel) & ~hi8);
-        const uint32_t hi = (__builtin_amdgcn_perm(H3, H2, sel) & hi8) | (__builtin_amdgcn_perm(H1, H0, sel) & ~hi8);
-        q01 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(hi, lo, 0x05010400u));
-        q23 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(hi, lo, 0x07030602u));
-    }
-    static __device__ __forceinline__ void bops(const Ch& c, int lane, const float (&wk)[2], half8 (&bf)[2][2]) {
-        uint32_t se[2][2], so[2][2];
-        GemmCodes<4>::spread(c.c, lane, se, so);
-        const auto st = __builtin_amdgcn_permlane32_swap(c.s0, c.s0, false, false);
-#pragma unroll
-        for (int T = 0; T < 2; ++T) {
-            const _Float16 sc = _Float16(__uint_as_float(st[T]) * wk[T]);
-            const half2v s2 = {sc, sc};
-#pragma unroll
-            for (int kk = 0; kk < 2; ++kk) {
-                half2v q[4];
-                look4(se[T][kk], q[0], q[1]);
-                look4(so[T][kk], q[2], q[3]);
-                uint32_t p[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) p[i] = __builtin_bit_cast(uint32_t, q[i] * s2);
-                bf[T][kk] = __builtin_bit_cast(half8, make_uint4(p[0], p[1], p[2], p[3]));
-            }
-        }
-    }
-};
 
 // Row factors (RplArgs::wrow) of row group g in the B-operand layout: wk[T]
 // belongs to row 32T + lane % 32, the lane's row in 32-row tile T. Two plain
@@ -1065,46 +714,6 @@ size_t gemm_scale_floats(int M) { return (size_t(M) + 63) / 64 * 64; }
 size_t gemm_scratch_floats(const DevBlob& b, int M) {
     const GemmPlan p = gemm_plan(b, M);
     return gemm_x_floats(b, M) + gemm_scale_floats(M) + (p.splits > 1 ? size_t(p.splits) * size_t(M) * size_t(b.rows) : 0);
-}
-
-// Calls go.template run<GP>() with the B-operand builder of b's format.
-template <class Go>
-int with_builder(const DevBlob& b, const Go& go) {
-    switch (b.fmt) {
-    case FMT_Q2_K: go.template run<GemmKQ<2>>(); return 0;
-    case FMT_Q3_K: go.template run<GemmKQ<3>>(); return 0;
-    case FMT_Q4_K: go.template run<GemmKQ<4>>(); return 0;
-    case FMT_Q5_K: go.template run<GemmKQ<5>>(); return 0;
-    case FMT_Q6_K: go.template run<GemmQ6>(); return 0;
-    case FMT_Q8_0: go.template run<GemmQ8>(); return 0;
-    case FMT_Q4_0: go.template run<GemmB32<4, false, 8, 0x88888888u>>(); return 0;
-    case FMT_Q4_1: go.template run<GemmB32<4, true, 0, 0u>>(); return 0;
-    case FMT_Q5_0: go.template run<GemmB32<5, false, 16, 0u>>(); return 0;
-    case FMT_Q5_1: go.template run<GemmB32<5, true, 0, 0u>>(); return 0;
-    case FMT_AFFINE:
-        switch (b.block_weights) {
-        case 32: go.template run<GemmB32<4, true, 0, 0u, 0>>(); return 0;
-        case 64: go.template run<GemmB32<4, true, 0, 0u, 1>>(); return 0;
-        case 128: go.template run<GemmB32<4, true, 0, 0u, 2>>(); return 0;
-        case 256: go.template run<GemmB32<4, true, 0, 0u, 3>>(); return 0;
-        default: return int(hipErrorInvalidValue);
-        }
-    case FMT_BINARY:
-        if (b.block_weights == 128) {
-            go.template run<GemmLin<1, false, 1, 2>>();
-            return 0;
-        }
-        [[fallthrough]];
-    case FMT_IQ1_S: go.template run<GemmLin<1, false, 1>>(); return 0;
-    case FMT_IQ2_XXS: go.template run<GemmLin<2, false, 3>>(); return 0;
-    case FMT_IQ2_XS: go.template run<GemmLin<2, true, 3>>(); return 0;
-    case FMT_IQ3_XXS: go.template run<GemmLin<3, false, 7>>(); return 0;
-    case FMT_IQ3_S: go.template run<GemmLin<3, true, 7>>(); return 0;
-    case FMT_IQ4_XS: go.template run<GemmLin<4, true, 15>>(); return 0;
-    case FMT_TERNARY: go.template run<GemmLin<2, true, 2>>(); return 0;
-    case FMT_IQ4_NL: go.template run<GemmNL>(); return 0;
-    default: return int(hipErrorInvalidValue);
-    }
 }
 
 // k_gemm_q4k_pw with TM 32-token tiles per wave; WF: apply the row factors.

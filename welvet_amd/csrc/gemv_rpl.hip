@@ -1738,8 +1738,14 @@ int launch_rpl_ex(const DevBlob& b, const float* d_x, float* d_y, int batch, voi
     }
 }
 
+void launch_rpl_ksum(const RplArgs& a, float* y, int batch, void* stream) {
+    hipLaunchKernelGGL(k_rpl_ksum, dim3(unsigned(a.rg_count), unsigned(batch)), dim3(64), 0,
+                       static_cast<hipStream_t>(stream), a, y);
+}
+
 int launch_rpl(const DevBlob& b, const float* d_x, float* d_y, int batch, void* stream, int mode, const float* aux,
                float* d_scratch) {
+    if (mode == RPL_STORE && gemv_b_supported(b, batch)) return launch_gemv_b(b, d_x, d_y, batch, stream, d_scratch);
     RplExtra ex;
     ex.mode = mode;
     ex.aux = aux;
@@ -1967,6 +1973,12 @@ size_t rpl_t_scratch_floats(const RplArgs& a, int batch) {
 }
 
 size_t rpl_scratch_floats(const DevBlob& b, int batch) {
+    if (b.layout != LAYOUT_RPL || batch <= 0) return 0;
+    if (gemv_b_supported(b, batch)) return gemv_b_scratch_floats(b, batch);
+    return rpl_rowwise_scratch_floats(b, batch);
+}
+
+size_t rpl_rowwise_scratch_floats(const DevBlob& b, int batch) {
     if (b.layout != LAYOUT_RPL || batch <= 0) return 0;
     const RplPlan p = rpl_plan(b, rpl_words2(b) ? 2 : 4);  // the plan launch_rpl_t makes for this blob
     if (p.ksplit <= 1) return 0;

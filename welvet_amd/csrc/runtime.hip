@@ -992,8 +992,10 @@ int wv_matvec_dev_noalloc(uint64_t handle, const float* d_x, float* d_y, int32_t
     }
     if (!sp) return fail(WV_E_NODEV, "MatVec (no-alloc): device %d has no scratch (not initialised)", b.device);
     // Every partial the split kernels read was written earlier in the same
-    // call, so the array needs no clearing between calls.
-    const size_t need = matvec_scratch_floats(b, batch);
+    // call, so the array needs no clearing between calls. A call is held to
+    // the one-row kernels' partials whichever kernel runs it; the batched
+    // kernel's (at most 2^18 floats) fit the array as well.
+    const size_t need = std::max(rpl_rowwise_scratch_floats(b, batch), matvec_scratch_floats(b, batch));
     if (need > kNoAllocScratchFloats)
         return fail(WV_E_SHAPE, "MatVec (no-alloc): rows=%lld cols=%lld needs %zu floats of scratch, the fixed array holds %zu",
                     (long long)b.rows, (long long)b.cols, need, kNoAllocScratchFloats);

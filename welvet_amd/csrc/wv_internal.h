@@ -265,6 +265,16 @@ int launch_rpl(const DevBlob& b, const float* d_x, float* d_y, int batch, void* 
                const float* aux = nullptr, float* d_scratch = nullptr);
 int launch_rpl_ex(const DevBlob& b, const float* d_x, float* d_y, int batch, void* stream, const RplExtra& ex);
 size_t rpl_scratch_floats(const DevBlob& b, int batch);
+// The partials of a batch on the one-row kernels, 8 rows per K-split launch:
+// what wv_matvec_dev_noalloc holds a call to.
+size_t rpl_rowwise_scratch_floats(const DevBlob& b, int batch);
+// Adds a K-split launch's partials in split order and stores (a.mode) y.
+void launch_rpl_ksum(const RplArgs& a, float* y, int batch, void* stream);
+// The batched forward at f32 precision (gemv_batch.hip), 2 rows and more of
+// every row-interleaved format but IQ4_NL. At most 2^18 floats of partials.
+bool gemv_b_supported(const DevBlob& b, int batch);
+size_t gemv_b_scratch_floats(const DevBlob& b, int batch);
+int launch_gemv_b(const DevBlob& b, const float* d_x, float* d_y, int batch, void* stream, float* d_scratch);
 size_t matvec_scratch_floats(const DevBlob& b, int batch);
 int launch_matvec(const DevBlob& b, const float* d_x, float* d_y, int batch, void* stream, float* d_scratch,
                   const BiasAct* ba = nullptr);
