@@ -277,3 +277,26 @@ def test_prefill_reference_layout_uses_batched_gemv(fmt, cols, force_raw):
     ref = oracle.reference_y(op, x)
     assert normwise(d.matmul(x), ref) <= TOL_F32
     d.free()
+
+
+@pytest.mark.parametrize("fmt", ["Q4_K", "Q6_K", "Q8_0", "Q4_1", "IQ2_XS"])
+@pytest.mark.parametrize("m,cols", [(1793, 256), (2048, 768)])
+def test_prefill_256_token_tiles(fmt, m, cols):
+    """Blocks long enough for 256-token tiles (20 row tiles x 8 token tiles fill
+    the GPU once where 128-token tiles take two passes): one and three
+    super-blocks, a last tile of one token, a ragged last row group, and a row
+    of tiny weights that brings in the kernel with the row factors."""
+    rows = 5001
+    print(f"[gpu] prefill 256-token tiles {fmt} {cols}->{rows} M={m}", flush=True)
+    rng = np.random.default_rng(m + cols)
+    w = (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32)
+    w[7] *= np.float32(1e-6)
+    p = wv.pack(fmt, w.reshape(-1), rows, cols)
+    d = wv.upload(p)
+    x = rng.standard_normal((m, cols)).astype(np.float32)
+    wd = oracle.unpack(oracle.Packed(p.fmt, rows, cols, p.raw, p.scales, p.meta, p.block_weights, p.mins))
+    ref = x.astype(np.float64) @ wd.reshape(rows, cols).astype(np.float64).T
+    y = d.matmul(x)
+    assert normwise(y, ref) <= TOL_MFMA
+    assert normwise(y[:, 7], ref[:, 7]) <= 4 * TOL_MFMA  # the tiny row on its own: fp16's precision, not subnormal
+    d.free()

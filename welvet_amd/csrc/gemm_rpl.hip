@@ -34,6 +34,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 #include "rpl_operands.h"
 #include "wave_ops.h"
@@ -360,16 +361,27 @@ __global__ void __launch_bounds__(1024) k_norm_x_f16r(float* __restrict__ h, con
 // LDS carries X alone: per K-step a block writes 16 KB of fp16 X and each
 // wave reads 16 KB back for 32 MFMAs (128 tokens x 64 rows x 64 columns),
 // against 96 KB per 16 MFMAs per wave with fp16 W tiles.
+// One wave per SIMD, so its LDS round trips are its own to hide: reading the A
+// fragments a k16 step ahead (and X a step ahead of that, in three buffers)
+// took Q4_K 4096->14336 from 81 to 75 us at M = 512, and 256-token tiles
+// (TM = 8) from 302 to 268 at M = 2047; the register rings as named values or
+// native vectors (the compiler kept a ring of structs in memory for Q8_0 and
+// Q4_0) took Q8_0 M = 512 from 139 to 82, Q4_0 4096->4096 from 64 to 41. What
+// bounds it now: 900 TFLOP/s at M = 2047, where the same loop without A reads
+// and without dequantization runs 1060 and a register-only loop of these MFMAs
+// on random data 1780 over 300 us (the clock gives way: 2150 over 2.5 ms);
+// 448 tiles take two passes of 256 CUs.
 template <class GP, int TM, int D, bool WF>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) k_gemm_q4k_pw(GemmArgs ga) {
     constexpr int BM = 32 * TM;
     constexpr int XB = BM * (BK / 8) / 256;  // 8-column X blocks per thread per K-step
     static_assert(XB >= 1 && 4 % D == 0, "shape");
-    __shared__ __attribute__((aligned(16))) _Float16 xs[2][BM * LDK];
+    __shared__ __attribute__((aligned(16))) _Float16 xs[3][BM * LDK];
     __shared__ float xsc[BM];  // the tile's row factors, for the epilogue
 
     const RplArgs& a = ga.w;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // wave-uniform: chunk addresses stay scalar
     const int nblk = blockIdx.x, mblk = blockIdx.y, split = blockIdx.z;
     const int sb0 = split * ga.sb_per_split;
     const int sb1 = min(a.nsb, sb0 + ga.sb_per_split);
@@ -382,24 +394,40 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     float wk[2] = {1.0f, 1.0f};  // row factors of the lane's rows in the two 32-row tiles
     if constexpr (WF) row_factors(a, g, lane, wk);
 
-    struct Regs {
+    struct Codes {
         typename GP::Ch c[2];  // the step's two chunks of this lane's row
-        uint4 xv[XB];          // fp16 X blocks
     };
-    auto load = [&](int s, Regs& r) {
-        const int sb = sb0 + s / 4;
-        const int64_t si = int64_t(g) * a.nsb + sb;
+    struct Xv {
+        u32x4 v[XB];  // fp16 X blocks of one K-step
+    };
+    auto load_c = [&](int s, Codes& r) {
+        const int64_t si = int64_t(g) * a.nsb + sb0 + s / 4;
 #pragma unroll
         for (int jj = 0; jj < 2; ++jj) {
             const int j = 2 * (s & 3) + jj;
             r.c[jj] = GP::load(a, rpl_chunk(a, si, j), si, j, lane);
         }
-        const int k8 = sb * 32 + (s & 3) * 8;
+    };
+    // this thread's blocks: rows t / 8 + 32 i of the tile, block t % 8 of the step
+    int xoff[XB];
 #pragma unroll
-        for (int i = 0; i < XB; ++i) {
-            const int f = t + 256 * i, m = min(mblk * BM + f / 8, ga.M - 1);
-            r.xv[i] = ga.xh[int64_t(m) * kb8 + k8 + f % 8];
-        }
+    for (int i = 0; i < XB; ++i) xoff[i] = (min(mblk * BM + t / 8 + 32 * i, ga.M - 1) - mblk * BM) * kb8;
+    const u32x4* xsrc = reinterpret_cast<const u32x4*>(ga.xh) + int64_t(mblk) * BM * kb8 + sb0 * 32 + t % 8;
+    auto load_x = [&](int s) {
+        Xv r;
+#pragma unroll
+        for (int i = 0; i < XB; ++i) r.v[i] = xsrc[xoff[i] + 8 * s];
+        return r;
+    };
+    auto put_x = [&](int buf, const Xv& r) {
+        _Float16* p = &xs[buf][(t / 8) * LDK + 8 * (t % 8)];
+#pragma unroll
+        for (int i = 0; i < XB; ++i) *reinterpret_cast<u32x4*>(p + 32 * i * LDK) = r.v[i];
+    };
+    auto read_a = [&](int buf, int ks, half8 (&af)[TM]) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+            af[i] = *reinterpret_cast<const half8*>(&xs[buf][(i * 32 + (lane & 31)) * LDK + ks * 16 + 8 * (lane >> 5)]);
     };
 
     f32x16 acc[TM][2];
@@ -410,57 +438,83 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-    Regs ring[D];
+    Codes cr[D];
+    // X of even and odd steps, in named registers: an indexed pair goes to memory
+    Xv xa = load_x(0), xb = load_x(min(1, steps - 1));
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-        load(min(d, steps - 1), ring[d]);
+        load_c(min(d, steps - 1), cr[d]);
         __builtin_amdgcn_sched_barrier(0);
     }
+    put_x(0, xa);
+    put_x(1, xb);
+    xa = load_x(min(2, steps - 1));
+    if constexpr (TM < 8) xb = load_x(min(3, steps - 1));
     // B operands: [chunk][tile][k16 step] as fp16 in k order [0,2,4,6,1,3,5,7].
-    // Step s + 1's are built (VALU) after the barrier, beside step s's MFMAs,
-    // so the matrix cores run while the next weights are dequantized.
+    // Step s + 1's are built (VALU) beside step s's MFMAs.
     half8 bf[2][2][2];
-    GP::bops(ring[0].c[0], lane, wk, bf[0]);
-    GP::bops(ring[0].c[1], lane, wk, bf[1]);
-    for (int s0 = 0; s0 < steps; s0 += D) {
+    GP::bops(cr[0].c[0], lane, wk, bf[0]);
+    GP::bops(cr[0].c[1], lane, wk, bf[1]);
+    load_c(min(D, steps - 1), cr[0]);
+    __syncthreads();
+    // One wave per SIMD: nothing else covers an LDS round trip, so the A
+    // fragments of each k16 step are read one k16 step ahead, across the step
+    // boundary too: X sits in three buffers (step s reads s and s + 1 and
+    // writes s + 2, whose readers of step s - 1 the last barrier has passed).
+    half8 a0[TM], a1[TM];
+    read_a(0, 0, a0);
+    int b0 = 0, b1 = 1, b2 = 2;  // buffers of steps s, s + 1, s + 2
+    auto mfmas = [&](const half8 (&af)[TM], const half8 (&b)[2][2], int kk) {
+        __builtin_amdgcn_sched_barrier(0x6);  // VALU and SALU may cross
 #pragma unroll
-        for (int d = 0; d < D; ++d) {
-            const int s = s0 + d, buf = s & 1;
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int i = 0; i < XB; ++i) {
-                const int f = t + 256 * i;
-                *reinterpret_cast<uint4*>(&xs[buf][(f / 8) * LDK + 8 * (f % 8)]) = ring[d].xv[i];
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            load(min(s + D, steps - 1), ring[d]);
-            __builtin_amdgcn_sched_barrier(0);
-            __syncthreads();
-            half8 bn[2][2][2];  // step s + 1 (its codes sit in the next ring slot)
-            GP::bops(ring[(d + 1) % D].c[0], lane, wk, bn[0]);
-            GP::bops(ring[(d + 1) % D].c[1], lane, wk, bn[1]);
-#pragma unroll
-            for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-                for (int kk = 0; kk < 2; ++kk) {
-                    const int ks = 2 * jj + kk;
-                    half8 af[TM];
-#pragma unroll
-                    for (int i = 0; i < TM; ++i)
-                        af[i] = *reinterpret_cast<const half8*>(
-                            &xs[buf][(i * 32 + (lane & 31)) * LDK + ks * 16 + 8 * (lane >> 5)]);
-#pragma unroll
-                    for (int i = 0; i < TM; ++i)
-#pragma unroll
-                        for (int T = 0; T < 2; ++T)
-                            acc[i][T] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[jj][T][kk], acc[i][T], 0, 0, 0);
-                }
-#pragma unroll
-            for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-                for (int T = 0; T < 2; ++T)
-#pragma unroll
-                    for (int kk = 0; kk < 2; ++kk) bf[jj][T][kk] = bn[jj][T][kk];
+            for (int T = 0; T < 2; ++T)
+                acc[i][T] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], b[T][kk], acc[i][T], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0x6);
+    };
+    auto step = [&](auto E, int s) {
+        constexpr int e = decltype(E)::value;
+        Codes& c = cr[(e + 1) % D];
+        half8 bn[2][2][2];  // step s + 1
+        read_a(b0, 1, a1);
+        if constexpr (TM == 8) {
+            put_x(b2, xa);
+            xa = load_x(min(s + 3, steps - 1));
+        } else if constexpr (e & 1) {
+            put_x(b2, xb);
+            xb = load_x(min(s + 4, steps - 1));
+        } else {
+            put_x(b2, xa);
+            xa = load_x(min(s + 4, steps - 1));
         }
+        mfmas(a0, bf[0], 0);
+        read_a(b0, 2, a0);
+        GP::bops(c.c[0], lane, wk, bn[0]);
+        mfmas(a1, bf[0], 1);
+        read_a(b0, 3, a1);
+        GP::bops(c.c[1], lane, wk, bn[1]);
+        load_c(min(s + 1 + D, steps - 1), c);
+        mfmas(a0, bf[1], 0);
+        read_a(b1, 0, a0);
+        mfmas(a1, bf[1], 1);
+        __syncthreads();
+#pragma unroll
+        for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+            for (int T = 0; T < 2; ++T)
+#pragma unroll
+                for (int kk = 0; kk < 2; ++kk) bf[jj][T][kk] = bn[jj][T][kk];
+        const int bt = b0;
+        b0 = b1;
+        b1 = b2;
+        b2 = bt;
+    };
+    for (int s0 = 0; s0 < steps; s0 += 4) {
+        step(std::integral_constant<int, 0>{}, s0);
+        step(std::integral_constant<int, 1>{}, s0 + 1);
+        step(std::integral_constant<int, 2>{}, s0 + 2);
+        step(std::integral_constant<int, 3>{}, s0 + 3);
     }
 
     // C[i][j] of a 32x32 tile: lane holds j = lane % 32, i = 8*(r/4) + 4*(lane/32) + r%4.
@@ -662,8 +716,8 @@ bool gemm_supported(const DevBlob& b, int M) {
 //   * 65 to 128 tokens on fewer row groups: k_gemm_rg with two 64-token
 //     blocks (8 waves, 2 per SIMD), K split as above (14336->4096 M = 128
 //     42.1-42.7 against 42.7-43.4 us on k_gemm_q4k_pw split 14 ways);
-//   * otherwise k_gemm_q4k_pw (256-row tiles of 128 tokens, one block per
-//     CU), K split while whole tiles leave CUs idle.
+//   * otherwise k_gemm_q4k_pw (256-row tiles of 128 or 256 tokens, one block
+//     per CU), K split while whole tiles leave CUs idle.
 enum { GEMM_PW = 1, GEMM_RG = 2 };
 // k_gemm_rg waves per block: 8 (2 per SIMD) for one or two 32-token tiles,
 // 4 (1 per SIMD) for four.
@@ -673,6 +727,7 @@ struct GemmPlan {
 };
 constexpr int kRgMinBlocks = 200;  // row groups on which 128-token k_gemm_rg blocks fill the GPU unsplit
 constexpr int64_t kCUs = 256;       // MI355X
+int64_t pw_passes(int64_t tiles) { return (tiles + kCUs - 1) / kCUs; }  // of the GPU, one block per CU
 GemmPlan gemm_plan(const DevBlob& b, int M) {
     const RplArgs& a = b.rpl;
     GemmPlan p{GEMM_PW, M <= 32 ? 32 : M <= 64 || (M <= 128 && a.rg_count < kRgMinBlocks) ? 64 : 128, 1, a.nsb, 1, 1};
@@ -695,7 +750,11 @@ GemmPlan gemm_plan(const DevBlob& b, int M) {
             }
         }
     } else {
-        const int64_t tiles = int64_t((a.rows + 255) / 256) * ((M + p.bm - 1) / p.bm);
+        const int64_t nrow = (a.rows + 255) / 256;
+        // 256-token tiles dequantize half as often per product and take 1.82 times a 128-token tile
+        // (4096->14336: 131 against 72 us a pass): where that beats the 128-token grid's passes.
+        if (1.85 * double(pw_passes(nrow * ((M + 255) / 256))) < double(pw_passes(nrow * ((M + 127) / 128)))) p.bm = 256;
+        const int64_t tiles = nrow * ((M + p.bm - 1) / p.bm);
         want = int(std::max<int64_t>(1, 256 / tiles));
         want = std::min(want, std::max(1, a.nsb / 2));  // each split >= 2 super-blocks
     }
@@ -727,7 +786,7 @@ struct PwGo {
     const GemmArgs& ga;
     template <class GP>
     void run() const {
-        hipLaunchKernelGGL((k_gemm_q4k_pw<GP, TM, 4, WF>), grid, dim3(256), 0, s, ga);
+        hipLaunchKernelGGL((k_gemm_q4k_pw<GP, TM, TM == 8 ? 2 : 4, WF>), grid, dim3(256), 0, s, ga);
     }
 };
 
@@ -756,7 +815,7 @@ int launch_tiles(const DevBlob& b, const GemmPlan& p, dim3 grid, hipStream_t s, 
         return p.bm == 32   ? with_builder(b, RgGo<1, WF>{grid, p.W, p.per, s, ga})
                : p.bm == 64 ? with_builder(b, RgGo<2, WF>{grid, p.W, p.per, s, ga})
                             : with_builder(b, RgGo<4, WF>{grid, p.W, p.per, s, ga});
-    return with_builder(b, PwGo<4, WF>{grid, s, ga});
+    return p.bm == 256 ? with_builder(b, PwGo<8, WF>{grid, s, ga}) : with_builder(b, PwGo<4, WF>{grid, s, ga});
 }
 
 bool gemm_x_frag(const DevBlob& b, int M) { return gemm_plan(b, M).kind == GEMM_RG; }
