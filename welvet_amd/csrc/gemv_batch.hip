@@ -412,16 +412,17 @@ struct GemvBGo {
 
 // A launch takes 9-13 us however few weights it has (a wave's chain of x,
 // conversion and chunks, and the K split's second launch on few rows), where
-// the one-row kernels take 5-6 us plus 0.08 us (integer dots) to 0.18 us (the
-// float dots of Q6_K and Q8_0) per million weights and batch row. Measured
-// crossings, weights x rows: Q4_K 4096x4096 at 5 rows (84 M; 9.5 against
-// 9.7 us at 4), Q6_K at 4, Q8_0 at 3 (50 M; 9.8 against 9.2 at 2), 1024x4096
-// Q4_K between 16 and 32 rows; 14336x4096 from 2 rows (12.9 against 13.9).
-// IQ4_NL's float grid is not exact in fp16.
+// the one-row kernels take 4-5 us plus 0.07 us (Q8_0 0.12 or more) per million
+// weights and batch row. The lines are where both sides met on a grid of 9
+// shapes from 1024x4096 to 14336x4096 and 2 to 32 rows, weights x rows: Q4_K
+// 9.3 against 10.0 us here at 67 M, 13.2 against 12.6 at 94 M, 14.8 against
+// 11.4 at 126 M; Q6_K and Q4_0 alike; Q8_0 8 rows and fewer 13.3 against 12.1
+// at 44 M, 15.4 against 10.0 at 67 M, more rows 10.9 against 11.8 at 67 M, 14.1
+// against 10.4 at 94 M. IQ4_NL's float grid is not exact in fp16.
 bool gemv_b_supported(const DevBlob& b, int batch) {
     const double work = double(batch) * double(b.rows) * double(b.cols);
-    const bool float_dots = b.fmt == FMT_Q6_K || b.fmt == FMT_Q8_0;
-    return batch >= 2 && b.layout == LAYOUT_RPL && b.fmt != FMT_IQ4_NL && work >= (float_dots ? 56e6 : 84e6);
+    const double line = b.fmt != FMT_Q8_0 ? 105e6 : batch <= 8 ? 60e6 : 90e6;
+    return batch >= 2 && b.layout == LAYOUT_RPL && b.fmt != FMT_IQ4_NL && work >= line;
 }
 
 size_t gemv_b_scratch_floats(const DevBlob& b, int batch) {
