@@ -291,3 +291,39 @@ def test_decoder_output_replaced_after_capture():
         rl, _ = ref.step(7, 20)
         assert normwise(got, rl) <= TOL
     dec.free()
+
+
+@pytest.mark.parametrize("rows,batch", [(7, 1), (1001, 1), (262144 - 256 - 64, 1), (262144, 1), (300, 200), (300, 600)])
+def test_host_staging_sizes(rows, batch):
+    """Host calls whose buffers fit the pinned bounce slot, end with it (256
+    columns of x and these rows fill 1 MiB), pass it, and mix both (the input
+    in the slot, the output from the pool): every value comes back, from first
+    calls and repeated ones, and the caller's x is left as it was."""
+    rng = np.random.default_rng(rows + batch)
+    w = (rng.standard_normal(rows * 256) * 0.02).astype(np.float32)
+    p = wv.pack("Q8_0", w, rows, 256)
+    d = wv.upload(p)
+    for _ in range(3):
+        x = rng.standard_normal((batch, 256)).astype(np.float32)
+        kept = x.copy()
+        y = d.matvec(x)
+        assert normwise(y, oracle.reference_y(packed_ref(p), x)) <= TOL
+        assert np.array_equal(x, kept)
+    d.free()
+
+
+def test_host_calls_from_more_threads_than_bounce_slots():
+    p, d, rng = make("Q6_K", 2048, 1024, 12)
+    xs = rng.standard_normal((16, 1024)).astype(np.float32)
+    refs = oracle.reference_y(packed_ref(p), xs)
+    bad = []
+
+    def work(i):
+        for _ in range(20):
+            if normwise(d.matvec(xs[i]), refs[i]) > TOL:
+                bad.append(i)
+    th = [threading.Thread(target=work, args=(i,)) for i in range(16)]
+    [t.start() for t in th]
+    [t.join() for t in th]
+    assert not bad
+    d.free()

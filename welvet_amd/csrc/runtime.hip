@@ -218,15 +218,85 @@ struct CallScratch {
     }
 };
 
-// Device copies of a host call's buffers on stream s; finish() frees them in
-// stream order and waits for the stream.
+// Bounce slots of the host entry points: a pinned host buffer and a device
+// buffer of kStageBytes each, at most kStageSlots per device, made on first
+// use, held by one call at a time and kept for the process. A call that finds
+// none free, or needs more, stages through the pool below instead.
+constexpr size_t kStageBytes = size_t(1) << 20;
+constexpr int kStageSlots = 4;
+struct StageSlot {
+    uint8_t* host = nullptr;
+    uint8_t* dev = nullptr;
+    bool busy = false;
+};
+struct DeviceStage {
+    std::mutex mu;
+    StageSlot slot[kStageSlots];
+};
+DeviceStage g_stage[64];
+
+// n 4-byte words between a bounce slot's pinned and device buffers (both
+// 256-byte aligned), as a kernel in the call's own queue: a copy engine's
+// transfer of a few KB waits for signals on both sides.
+__global__ void __launch_bounds__(256) k_stage_copy(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src, size_t n) {
+    const size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;
+    if (4 * i + 4 <= n) {
+        reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
+    } else {
+        for (size_t k = 4 * i; k < n; ++k) dst[k] = src[k];
+    }
+}
+
+// Device copies of a host call's buffers on stream s; finish() waits for the
+// stream and releases them. Small buffers (all of a one-row call's) go through
+// a bounce slot: the host copies into pinned memory and k_stage_copy moves it,
+// and results come back the same way, the last host copy after the wait. A
+// pageable copy and a stream-ordered allocation per buffer took 62 us beside
+// the 19 us of the Q6_K 32000 x 4096 product. Larger ones are allocated from
+// the pool and copied by the runtime.
 struct Staging {
     hipStream_t s;
     std::vector<void*> bufs;
     hipError_t err = hipSuccess;
-    explicit Staging(hipStream_t st) : s(st) {}
+    StageSlot* sl = nullptr;
+    size_t used = 0;
+    struct Back {
+        void* h;
+        size_t off, bytes;
+    };
+    std::vector<Back> backs;
+    Staging(hipStream_t st, int dev) : s(st) {
+        if (dev < 0 || dev >= 64) return;
+        DeviceStage& ds = g_stage[dev];
+        std::lock_guard<std::mutex> lk(ds.mu);
+        for (StageSlot& c : ds.slot) {
+            if (c.busy) continue;
+            if (!c.host) {
+                void *h = nullptr, *d = nullptr;
+                if (hipHostMalloc(&h, kStageBytes, hipHostMallocDefault) != hipSuccess ||
+                    hipMalloc(&d, kStageBytes) != hipSuccess) {
+                    (void)hipGetLastError();  // the pool serves the call
+                    if (h) (void)hipHostFree(h);
+                    break;
+                }
+                c.host = static_cast<uint8_t*>(h);
+                c.dev = static_cast<uint8_t*>(d);
+            }
+            c.busy = true;
+            sl = &c;
+            mu = &ds.mu;
+            break;
+        }
+    }
+    Staging(const Staging&) = delete;
+    Staging& operator=(const Staging&) = delete;
     template <class T = float>
     T* out(size_t n) {
+        if (err == hipSuccess && sl && std::max<size_t>(n, 1) <= (kStageBytes - used) / sizeof(T)) {
+            T* p = reinterpret_cast<T*>(sl->dev + used);
+            used = std::min(kStageBytes, (used + std::max<size_t>(n, 1) * sizeof(T) + 255) & ~size_t(255));
+            return p;
+        }
         void* p = nullptr;
         if (err == hipSuccess) err = pool_alloc(&p, std::max<size_t>(n, 1) * sizeof(T), s);
         if (err == hipSuccess) bufs.push_back(p);
@@ -235,13 +305,27 @@ struct Staging {
     template <class T>
     T* in(const T* h, size_t n) {
         T* p = out<T>(n);
-        if (err == hipSuccess && n) err = hipMemcpyAsync(p, h, n * sizeof(T), hipMemcpyHostToDevice, s);
+        if (err != hipSuccess || !n) return p;
+        if (in_slot(p)) {
+            const size_t off = size_t(reinterpret_cast<uint8_t*>(p) - sl->dev);
+            std::memcpy(sl->host + off, h, n * sizeof(T));
+            copy(sl->dev + off, sl->host + off, n * sizeof(T));
+        } else {
+            err = hipMemcpyAsync(p, h, n * sizeof(T), hipMemcpyHostToDevice, s);
+        }
         return p;
     }
     int rc(const char* what) { return err == hipSuccess ? WV_OK : hip_fail(err, what); }
     template <class T>
     int back(T* h, const T* d, size_t n, const char* what) {
-        const hipError_t e = n ? hipMemcpyAsync(h, d, n * sizeof(T), hipMemcpyDeviceToHost, s) : hipSuccess;
+        if (!n) return WV_OK;
+        if (in_slot(d)) {
+            const size_t off = size_t(reinterpret_cast<const uint8_t*>(d) - sl->dev);
+            copy(sl->host + off, sl->dev + off, n * sizeof(T));
+            backs.push_back({h, off, n * sizeof(T)});
+            return err == hipSuccess ? WV_OK : hip_fail(err, what);
+        }
+        const hipError_t e = hipMemcpyAsync(h, d, n * sizeof(T), hipMemcpyDeviceToHost, s);
         return e == hipSuccess ? WV_OK : hip_fail(e, what);
     }
     int finish(int rc, const char* what) {
@@ -249,10 +333,37 @@ struct Staging {
         bufs.clear();
         const hipError_t e = hipStreamSynchronize(s);
         if (!rc && e != hipSuccess) rc = hip_fail(e, what);
+        if (!rc)
+            for (const Back& b : backs) std::memcpy(b.h, sl->host + b.off, b.bytes);
+        release();
         return rc;
     }
     ~Staging() {
         for (void* p : bufs) (void)hipFreeAsync(p, s);
+        if (sl) {  // finish() was not reached: the GPU may still use the slot
+            (void)hipStreamSynchronize(s);
+            release();
+        }
+    }
+
+private:
+    std::mutex* mu = nullptr;
+    bool in_slot(const void* d) const {
+        const uint8_t* p = static_cast<const uint8_t*>(d);
+        return sl && p >= sl->dev && p < sl->dev + kStageBytes;
+    }
+    void copy(void* dst, const void* src, size_t bytes) {
+        const size_t n = bytes / 4;  // every element type is 4 or 8 bytes
+        hipLaunchKernelGGL(k_stage_copy, dim3(unsigned((n + 1023) / 1024)), dim3(256), 0, s, static_cast<uint32_t*>(dst),
+                           static_cast<const uint32_t*>(src), n);
+        const hipError_t e = hipGetLastError();
+        if (err == hipSuccess) err = e;
+    }
+    void release() {
+        if (!sl) return;
+        std::lock_guard<std::mutex> lk(*mu);
+        sl->busy = false;
+        sl = nullptr;
     }
 };
 
@@ -1080,7 +1191,7 @@ int wv_matmul(uint64_t handle, const float* x, float* y, int32_t m) {
     if (m <= 0) return m < 0 ? fail(WV_E_ARG, "MatMul: negative row count %d", m) : WV_OK;
     (void)hipSetDevice(b.device);
     hipStream_t s = g_dev[b.device].stream;
-    Staging st(s);
+    Staging st(s, b.device);
     float* dx = st.in(x, size_t(m) * size_t(b.cols));
     float* dy = st.out(size_t(m) * size_t(b.rows));
     int rc = st.rc("MatMul: staging");
@@ -1096,7 +1207,7 @@ int wv_matvec(uint64_t handle, const float* x, float* y, int32_t batch) {
     if (batch <= 0) return batch < 0 ? fail(WV_E_SHAPE, "MatVec: negative batch %d", batch) : WV_OK;
     (void)hipSetDevice(b.device);
     hipStream_t s = g_dev[b.device].stream;
-    Staging st(s);
+    Staging st(s, b.device);
     float* dx = st.in(x, size_t(batch) * size_t(b.cols));
     float* dy = st.out(size_t(batch) * size_t(b.rows));
     int rc = st.rc("MatVec: staging");
@@ -1112,7 +1223,7 @@ int wv_matvec_t(uint64_t handle, const float* gy, float* gx, int32_t batch) {
     if (batch <= 0) return batch < 0 ? fail(WV_E_SHAPE, "MatVecT: negative batch %d", batch) : WV_OK;
     (void)hipSetDevice(b.device);
     hipStream_t s = g_dev[b.device].stream;
-    Staging st(s);
+    Staging st(s, b.device);
     float* dg = st.in(gy, size_t(batch) * size_t(b.rows));
     float* dx = st.in(gx, size_t(batch) * size_t(b.cols));
     int rc = st.rc("MatVecT: staging");
@@ -1193,7 +1304,7 @@ static int dense_forward_host(uint64_t handle, const float* x, float* pre, float
     (void)hipSetDevice(b.device);
     hipStream_t s = g_dev[b.device].stream;
     const size_t n = size_t(batch) * size_t(b.rows);
-    Staging st(s);
+    Staging st(s, b.device);
     float* dx = st.in(x, size_t(batch) * size_t(b.cols));
     float* dpre = st.out(n);
     float* dpost = post ? st.out(n) : nullptr;
@@ -1244,7 +1355,7 @@ int wv_store_matvec(uint64_t handle, const double* x, size_t len_x, double* y, s
         if (int64_t(len_x) < b.cols || int64_t(len_y) < b.rows) return fail(WV_E_SHAPE, "weights: matvecF64 shape");
         (void)hipSetDevice(b.device);
         hipStream_t s = g_dev[b.device].stream;
-        Staging st(s);
+        Staging st(s, b.device);
         double* dx = st.in(x, size_t(b.cols));
         double* dy = st.out<double>(size_t(b.rows));
         int rc = st.rc("weights: staging");
@@ -1274,7 +1385,7 @@ int wv_store_matvec_t(uint64_t handle, const double* gy, size_t len_gy, double* 
         if (int64_t(len_gy) < b.rows || int64_t(len_gx) < b.cols) return fail(WV_E_SHAPE, "weights: matvecTF64 shape");
         (void)hipSetDevice(b.device);
         hipStream_t s = g_dev[b.device].stream;
-        Staging st(s);
+        Staging st(s, b.device);
         double* dg = st.in(gy, size_t(b.rows));
         double* dx = st.in(gx, size_t(b.cols));
         double* part = st.out<double>(std::max<size_t>(1, store_t_scratch_floats(b) / 2));
