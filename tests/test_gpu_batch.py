@@ -105,3 +105,33 @@ def test_batched_forward_route_keeps_the_result():
     y8, y2 = d.matvec(x), np.concatenate([d.matvec(x[i:i + 2]) for i in range(0, 8, 2)])
     assert rowwise(y8.astype(np.float64), y2) <= TOL
     d.free()
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+def test_batched_gradient_formats(fmt):
+    rows, cols = 4700, 2304  # a ragged last row group; 9 super-blocks over the 8 XCDs; one slice of 8 waves
+    print(f"[gpu] batched gradient {fmt}", flush=True)
+    p, d, rng = make(fmt, rows, cols, 21)
+    check_gradient(p, d, rng, 10)  # quartets of rows and two left over
+    d.free()
+
+
+@pytest.mark.parametrize("shape", [(29000, 256, 24), (14337, 4096, 3), (4097, 4096, 5), (1030, 6144, 16), (500, 14336, 9),
+                                   (65, 14336, 67), (64, 65536, 16), (14337, 512, 23)])
+def test_batched_gradient_tiles(shape):
+    """One slice and several; fewer row groups than 8 waves hold, a chain of more than 8 row groups a wave with a
+    ragged end; remainders of the 4 rows of a block and of the 16 of a launch."""
+    rows, cols, batch = shape
+    print(f"[gpu] batched gradient Q4_K {rows}x{cols} batch {batch}", flush=True)
+    p, d, rng = make("Q4_K", rows, cols, rows + batch)
+    check_gradient(p, d, rng, batch)
+    d.free()
+
+
+def check_gradient(p, d, rng, batch):
+    """gx += W^T gy to the f32 bar of wv_matvec_t on each row, gx not zeroed."""
+    gy = rng.standard_normal((batch, p.rows)).astype(np.float32)
+    gx = rng.standard_normal((batch, p.cols)).astype(np.float32)
+    w = oracle.unpack(oracle.Packed(p.fmt, p.rows, p.cols, p.raw, p.scales, p.meta, p.block_weights, p.mins))
+    want = gx + gy.astype(np.float64) @ w.reshape(p.rows, p.cols).astype(np.float64)
+    assert rowwise(d.matvec_t(gy, gx).astype(np.float64), want) <= TOL

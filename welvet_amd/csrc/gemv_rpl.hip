@@ -1513,6 +1513,45 @@ struct TIQ4NL : RplIQ4NL {
     }
 };
 
+// The last five levels of a 64-lane reduce-scatter: v[i] of lanes 0-31 is value
+// i's and of lanes 32-63 value 32 + i's partial sum; lane l ends with value
+// l's total. Every level runs on the VALU: lane swaps for 16, DPP for 8 (l ^ 8),
+// 4 (partner l ^ 7, which also differs in bit 2), 2 and 1.
+__device__ __forceinline__ float reduce_columns32(float* v, int lane) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = reduce_scatter16(v[i], v[i + 16]);
+    {
+        const bool hi = (lane & 8) != 0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float keep = hi ? v[i + 8] : v[i], send = hi ? v[i] : v[i + 8];
+            v[i] = keep + row_xor8(send);
+        }
+    }
+    {
+        const bool hi = (lane & 4) != 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float keep = hi ? v[i + 4] : v[i], send = hi ? v[i] : v[i + 4];
+            v[i] = keep + half_mirror(send);
+        }
+    }
+    {
+        const bool hi = (lane & 2) != 0;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const float keep = hi ? v[i + 2] : v[i], send = hi ? v[i] : v[i + 2];
+            v[i] = keep + quad_xor2(send);
+        }
+    }
+    {
+        const bool hi = (lane & 1) != 0;
+        const float keep = hi ? v[1] : v[0], send = hi ? v[0] : v[1];
+        v[0] = keep + quad_xor1(send);
+    }
+    return v[0];
+}
+
 // Column group of block x in XCD-aware order. Consecutive block ids go to
 // the 8 XCDs in turn, so x = 32q + 8jp + k gives super-block sb = 8q + k,
 // chunk pair jp: the four chunk pairs of a super-block (ids 8 apart) run on
@@ -1584,37 +1623,7 @@ __global__ void __launch_bounds__(1024) k_gemvt_rpl(RplArgs a, const float* __re
     // also differs in bit 2), 2 and 1.
 #pragma unroll
     for (int i = 0; i < 32; ++i) acc[i] = reduce_scatter32(acc[i], acc[i + 32]);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = reduce_scatter16(acc[i], acc[i + 16]);
-    {
-        const bool hi = (lane & 8) != 0;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float keep = hi ? acc[i + 8] : acc[i], send = hi ? acc[i] : acc[i + 8];
-            acc[i] = keep + row_xor8(send);
-        }
-    }
-    {
-        const bool hi = (lane & 4) != 0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float keep = hi ? acc[i + 4] : acc[i], send = hi ? acc[i] : acc[i + 4];
-            acc[i] = keep + half_mirror(send);
-        }
-    }
-    {
-        const bool hi = (lane & 2) != 0;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const float keep = hi ? acc[i + 2] : acc[i], send = hi ? acc[i] : acc[i + 2];
-            acc[i] = keep + quad_xor2(send);
-        }
-    }
-    {
-        const bool hi = (lane & 1) != 0;
-        const float keep = hi ? acc[1] : acc[0], send = hi ? acc[0] : acc[1];
-        acc[0] = keep + quad_xor1(send);
-    }
+    const float colsum = reduce_columns32(acc, lane);
     // Group offsets: column l is in local group l >> 4 = 2*bit5 + bit4; after
     // the two swap levels every lane of a 16-lane row adds up its row.
     off[0] = reduce_scatter32(off[0], off[2]);
@@ -1622,7 +1631,7 @@ __global__ void __launch_bounds__(1024) k_gemvt_rpl(RplArgs a, const float* __re
     const float o = row_sum16(reduce_scatter16(off[0], off[1]));
 
     // the block's waves, added in wave order
-    red[wave * 64 + lane] = acc[0] + o;
+    red[wave * 64 + lane] = colsum + o;
     __syncthreads();
     if (wave != 0) return;
     float total = 0.f;
@@ -1637,6 +1646,113 @@ __global__ void __launch_bounds__(1024) k_gemvt_rpl(RplArgs a, const float* __re
     // slices in slice order (a last-arriving-block tail costs more here than
     // the extra launch: its ticket round trips bypass the caches).
     part[(int64_t(b) * nslices + slice) * cols + col] = total;
+}
+
+// The batched form, NB = 4 gy rows at once: the one-row kernel above decodes
+// the weights again for each row of the batch. A block is one 32-column chunk
+// (4 x 32 column sums a lane, where a pair for one row took 64), one slice of
+// W * n row groups and NB rows; a weight's code is converted once and meets
+// the NB rows in an FMA each (205 VALU instructions per chunk and 4 rows, 64
+// per row there). 14336x4096 Q4_K, us: 3 / 8 / 16 rows 23.5 / 36.3 / 70 against
+// 32.3 / 57.9 / 111. VALU-bound: 22 us of 8 rows' 36 at one instruction per 4
+// cycles. Lane l ends with column l % 32 of rows 2s + l /
+// 32 for s = 0, 1. The lane sums are reduced after every 8 row groups: in one
+// chain of 28, 14336 rows came out 3.7e-7 from f64 against 2.9e-7, and as
+// slices of 64 row groups 8 rows took 47.5 us. Rows past the batch repeat its last one and go nowhere.
+template <class P, int NB>
+__global__ void __launch_bounds__(512) k_gemvt_rpl_b(RplArgs a, const float* __restrict__ gy, float* __restrict__ gx,
+                                                     float* __restrict__ part, int batch, int n) {
+    static_assert(NB == 4, "two rows per 64-lane reduction");
+    __shared__ float red[NB / 2][8 * 64];
+    const int W = blockDim.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    // ids 8 apart run on one XCD: a super-block's 8 chunks read its metadata through one L2
+    const int sb = (blockIdx.x >> 6) * 8 + (blockIdx.x & 7), j = (blockIdx.x >> 3) & 7;
+    if (sb >= a.nsb) return;  // uniform over the block
+    const int slice = blockIdx.y, b0 = blockIdx.z * NB, nb = min(NB, batch - b0);
+    const int nslices = gridDim.y;
+    const int g0 = (slice * W + wave) * n;
+    const int64_t cols = int64_t(a.nsb) * 256;
+
+    float acc[NB][32], off[NB][2];
+    float tot[NB / 2] = {0.f, 0.f};
+    struct Set {
+        typename P::Ch c;
+        typename P::TM tm;
+        float g0, g1, g2, g3;
+    };
+    const float* gyb = gy + int64_t(b0) * a.rows;
+    const int64_t r1 = nb > 1 ? a.rows : 0, r2 = nb > 2 ? 2 * int64_t(a.rows) : 0, r3 = nb > 3 ? 3 * int64_t(a.rows) : 0;
+    auto load = [&](int i) {
+        const int g = min(g0 + min(i, n - 1), a.rg_count - 1);
+        const int64_t si = int64_t(g) * a.nsb + sb;
+        Set st;
+        st.c = P::load_ch(a, rpl_chunk(a, si, j), lane);
+        st.tm = P::load_tm(a, si, lane, j >> 1);
+        const float* p = gyb + min(g * 64 + lane, a.rows - 1);
+        st.g0 = p[0];
+        st.g1 = p[r1];
+        st.g2 = p[r2];
+        st.g3 = p[r3];
+        return st;
+    };
+    auto run = [&](auto J) {
+        constexpr int jj = decltype(J)::value;
+        auto add = [&](int i, const Set& st) {
+            const bool in = i < n && (g0 + i) * 64 + lane < a.rows;  // row groups and rows past the end add 0
+            P::template tacc<jj>(st.c, st.tm, in ? st.g0 : 0.f, acc[0], off[0]);
+            P::template tacc<jj>(st.c, st.tm, in ? st.g1 : 0.f, acc[1], off[1]);
+            P::template tacc<jj>(st.c, st.tm, in ? st.g2 : 0.f, acc[2], off[2]);
+            P::template tacc<jj>(st.c, st.tm, in ? st.g3 : 0.f, acc[3], off[3]);
+        };
+        Set x = load(0), y = load(1);
+        for (int i0 = 0; i0 < n; i0 += 8) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                off[b][0] = off[b][1] = 0.f;
+#pragma unroll
+                for (int k = 0; k < 32; ++k) acc[b][k] = 0.f;
+            }
+            for (int i = i0; i < min(n, i0 + 8); i += 2) {
+                __builtin_amdgcn_sched_barrier(0);
+                add(i, x);
+                __builtin_amdgcn_sched_barrier(0);
+                x = load(i + 2);
+                __builtin_amdgcn_sched_barrier(0);
+                add(i + 1, y);
+                __builtin_amdgcn_sched_barrier(0);
+                y = load(i + 3);
+            }
+            // Per pair of rows, the reduce-scatter of k_gemvt_rpl: value 32 (row % 2) + column.
+#pragma unroll
+            for (int s = 0; s < NB / 2; ++s) {
+                float v[32];
+#pragma unroll
+                for (int k = 0; k < 32; ++k) v[k] = reduce_scatter32(acc[2 * s][k], acc[2 * s + 1][k]);
+                const float o0 = reduce_scatter32(off[2 * s][0], off[2 * s + 1][0]);
+                const float o1 = reduce_scatter32(off[2 * s][1], off[2 * s + 1][1]);
+                tot[s] += reduce_columns32(v, lane) + row_sum16(reduce_scatter16(o0, o1));
+            }
+        }
+    };
+    if (j & 1) run(std::integral_constant<int, 1>{});
+    else run(std::integral_constant<int, 0>{});
+
+#pragma unroll
+    for (int s = 0; s < NB / 2; ++s) red[s][wave * 64 + lane] = tot[s];
+    __syncthreads();
+    if (wave >= NB / 2) return;
+    const int s = wave, b = 2 * s + (lane >> 5);
+    float total = 0.f;
+    for (int w = 0; w < W; ++w) total += red[s][w * 64 + lane];
+    if (b >= nb) return;
+    const int64_t col = int64_t(sb) * 256 + j * 32 + (lane & 31);
+    if (nslices == 1) {
+        gx[int64_t(b0 + b) * cols + col] += total;
+        return;
+    }
+    part[(int64_t(b0 + b) * nslices + slice) * cols + col] = total;
 }
 
 // Row-group slices for `batch` rows. One slice (no second pass) when the
@@ -1667,12 +1783,52 @@ RplTPlan rpl_t_plan(const RplArgs& a, int batch) {
     return p;
 }
 
+// The batched form: one slice when the chunks and row quartets alone give at
+// least kRplTMinBlocks blocks, else slices for about kRplTBlocks; waves of at
+// least 8 row groups where there are as many (a wave's column reduction costs
+// as much as two of them), up to 8 waves.
+constexpr int kRplTBatch = 4;
+struct RplTBPlan {
+    int slices, W, n;
+};
+RplTBPlan rpl_tb_plan(const RplArgs& a, int batch) {
+    const int64_t per_slice = int64_t(a.nsb) * 8 * ((batch + kRplTBatch - 1) / kRplTBatch);
+    int64_t slices = 1;
+    if (per_slice < kRplTMinBlocks) slices = std::min<int64_t>((kRplTBlocks + per_slice - 1) / per_slice, a.rg_count);
+    const int64_t rps = (a.rg_count + slices - 1) / slices;
+    RplTBPlan p;
+    p.W = int(std::min<int64_t>(8, std::max<int64_t>(2, (rps + 7) / 8)));
+    p.n = int((rps + p.W - 1) / p.W);
+    p.slices = int((a.rg_count + int64_t(p.W) * p.n - 1) / (int64_t(p.W) * p.n));
+    return p;
+}
+// From 3 rows, where it runs as one slice (its chunks fill the GPU) with some
+// work, or has the work to pay for slices of a kernel this long: 4096x4096 Q6_K
+// 8 rows, one slice, 10.9 against 15.7 us; 4 rows, two slices (67 M weights x
+// rows), 11.2 against 9.4; Q4_K 14336x4096 3 rows, two slices (176 M), 23.5
+// against 32.3; one slice of 1024x14336, 4 rows (58 M) 11.9 against 10.8, 8 rows
+// 12.4 against 16.9; of 3072x7168 Q8_0, 3 rows (66 M) 11.2 against 20.0.
+bool rpl_t_batched(const RplArgs& a, int batch) {
+    const int64_t per_slice = int64_t(a.nsb) * 8 * ((batch + kRplTBatch - 1) / kRplTBatch);
+    const double work = double(batch) * double(a.rows) * double(a.nsb) * 256.0;
+    return batch >= kRplTBatch - 1 && work >= (per_slice >= kRplTMinBlocks ? 62e6 : 150e6);
+}
+
 template <class P>
 int launch_rpl_tr(const DevBlob& bl, const float* gy, float* gx, int batch, hipStream_t s, float* part) {
     const RplArgs& a = bl.rpl;
     const int64_t cols = int64_t(a.nsb) * 256;
     for (int b0 = 0; b0 < batch; b0 += kRplTMaxBatch) {
         const int nb = std::min(kRplTMaxBatch, batch - b0);
+        if (rpl_t_batched(a, nb)) {
+            const RplTBPlan p = rpl_tb_plan(a, nb);
+            if (p.slices > 1 && !part) return int(hipErrorInvalidValue);
+            const dim3 grid(unsigned((a.nsb + 7) / 8 * 64), unsigned(p.slices), unsigned((nb + kRplTBatch - 1) / kRplTBatch));
+            hipLaunchKernelGGL((k_gemvt_rpl_b<P, kRplTBatch>), grid, dim3(unsigned(64 * p.W)), 0, s, a,
+                               gy + int64_t(b0) * a.rows, gx + int64_t(b0) * cols, part, nb, p.n);
+            if (p.slices > 1) launch_gemvt_reduce(part, gx + int64_t(b0) * cols, cols, p.slices, nb, s);
+            continue;
+        }
         const RplTPlan p = rpl_t_plan(a, nb);
         auto kern = p.GP == 1 ? k_gemvt_rpl<P, 1> : p.GP == 2 ? k_gemvt_rpl<P, 2> : p.GP == 4 ? k_gemvt_rpl<P, 4> : k_gemvt_rpl<P, 8>;
         if (p.slices > 1 && !part) return int(hipErrorInvalidValue);  // the caller owes the slice scratch
@@ -1966,8 +2122,8 @@ size_t rpl_t_scratch_floats(const RplArgs& a, int batch) {
     const int full = std::min(batch, kRplTMaxBatch), rest = batch % kRplTMaxBatch;
     for (int nb : {full, rest}) {
         if (nb <= 0) continue;
-        const RplTPlan p = rpl_t_plan(a, nb);
-        if (p.slices > 1) most = std::max(most, size_t(p.slices) * size_t(nb) * size_t(a.nsb) * 256);
+        const int slices = rpl_t_batched(a, nb) ? rpl_tb_plan(a, nb).slices : rpl_t_plan(a, nb).slices;
+        if (slices > 1) most = std::max(most, size_t(slices) * size_t(nb) * size_t(a.nsb) * 256);
     }
     return most;
 }
