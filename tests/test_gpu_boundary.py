@@ -327,3 +327,20 @@ def test_host_calls_from_more_threads_than_bounce_slots():
     [t.join() for t in th]
     assert not bad
     d.free()
+
+
+@pytest.mark.parametrize("rows", [1024, 1022, 5, 1027])
+@pytest.mark.parametrize("act", ["linear", "relu", "silu", "gelu", "tanh", "sigmoid", "leaky_relu", "relu2"])
+def test_bias_act_large_blocks(rows, act):
+    """The epilogue on a million outputs (four columns a thread where rows are whole float4s) and on ragged rows:
+    pre and post from the library's own product, so to the rounding of f32(act(f64(pre)))."""
+    batch = 1100 if rows > 5 else 3
+    p, d, rng = make("Q8_0", rows, 256, rows)
+    x = rng.standard_normal((batch, 256)).astype(np.float32)
+    bias = rng.standard_normal(rows)
+    y = d.matvec(x)
+    pre, post = d.dense_forward(x, bias, act)
+    want_pre, want_post = dense_ref.apply_bias_act(y, bias, act)
+    assert np.array_equal(pre, np.asarray(want_pre, np.float32).reshape(pre.shape))
+    assert normwise(post, want_post) <= 1.2e-7  # one ulp of f32 (2^-23): the device's exp and tanh may round the other way
+    d.free()

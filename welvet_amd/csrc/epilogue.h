@@ -27,14 +27,4 @@ __device__ __forceinline__ double activate_f64(double x, int act) {
     }
 }
 
-// Stores pre (biased when `bias` is set) to y[idx] and act(pre) to post[idx];
-// returns the stored pre.
-__device__ __forceinline__ float store_bias_act(float* y, float* post, int64_t idx, float s, const double* bias,
-                                                int64_t row, int act) {
-    if (bias) s = float(double(s) + bias[row]);
-    y[idx] = s;
-    post[idx] = act == ACT_LINEAR ? s : float(activate_f64(double(s), act));
-    return s;
-}
-
 }  // namespace wv

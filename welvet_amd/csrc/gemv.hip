@@ -566,12 +566,41 @@ __global__ void __launch_bounds__(64) k_gemvt_reduce(const float* __restrict__ p
 // f32(y + bias) written to `pre`, post = f32(act(f64(pre))) to `post`. y and
 // pre may be the same buffer (in place; each thread reads its element before
 // writing it), so neither is declared __restrict__.
-__global__ void __launch_bounds__(256) k_bias_act(const float* y, float* pre,
-                                                  float* __restrict__ post, const double* __restrict__ bias, int act,
-                                                  int64_t rows, int64_t n) {
-    const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (i >= n) return;
-    store_bias_act(pre, post, i, y[i], bias, i % rows, act);
+// A thread owns V consecutive columns (V = 4: whole float4s) of every
+// gridDim.y-th batch row, its bias in registers. With one element per thread
+// and its column taken from a flat 64-bit index the division cost as much as
+// the activation: 2047 x 14336 with bias and SiLU 89 us, now 71, for 352 MB
+// (68 us at a large copy's 5.2 TB/s).
+template <int V>
+__global__ void __launch_bounds__(256) k_bias_act(const float* y, float* pre, float* __restrict__ post,
+                                                  const double* __restrict__ bias, int act, int64_t rows, int batch) {
+    const int64_t c = (int64_t(blockIdx.x) * 256 + threadIdx.x) * V;
+    if (c >= rows) return;
+    double bv[V];
+#pragma unroll
+    for (int k = 0; k < V; ++k) bv[k] = bias ? bias[c + k] : 0.0;
+    for (int b = blockIdx.y; b < batch; b += gridDim.y) {
+        const int64_t i = int64_t(b) * rows + c;
+        float v[V], o[V];
+        if constexpr (V == 4) {
+            const float4 t = *reinterpret_cast<const float4*>(y + i);
+            v[0] = t.x, v[1] = t.y, v[2] = t.z, v[3] = t.w;
+        } else {
+            v[0] = y[i];
+        }
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+            if (bias) v[k] = float(double(v[k]) + bv[k]);
+            o[k] = act == ACT_LINEAR ? v[k] : float(activate_f64(double(v[k]), act));
+        }
+        if constexpr (V == 4) {
+            *reinterpret_cast<float4*>(pre + i) = make_float4(v[0], v[1], v[2], v[3]);
+            *reinterpret_cast<float4*>(post + i) = make_float4(o[0], o[1], o[2], o[3]);
+        } else {
+            pre[i] = v[0];
+            post[i] = o[0];
+        }
+    }
 }
 
 RawArgs raw_args(const DevBlob& b) {
@@ -746,10 +775,19 @@ int launch_matvec(const DevBlob& b, const float* d_x, float* d_y, int batch, voi
 
 int launch_bias_act(const float* d_y, float* d_pre, float* d_post, const double* d_bias, int act, int64_t rows,
                     int batch, void* stream) {
-    const int64_t n = rows * int64_t(batch);
-    if (n == 0) return 0;
-    hipLaunchKernelGGL(k_bias_act, dim3(unsigned((n + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream), d_y,
-                       d_pre, d_post, d_bias, act, rows, n);
+    if (rows * int64_t(batch) == 0) return 0;
+    // float4s where the rows and buffers allow it and there are enough of them to fill the GPU
+    auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    const bool vec = rows % 4 == 0 && aligned(d_y) && aligned(d_pre) && aligned(d_post) &&
+                     rows * int64_t(batch) >= int64_t(1) << 20;
+    const int64_t gx = (rows / (vec ? 4 : 1) + 255) / 256;
+    const dim3 grid(unsigned(gx), unsigned(std::min<int64_t>(batch, vec ? std::max<int64_t>(1, 8192 / gx) : 65535)));
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, grid, dim3(256), 0, static_cast<hipStream_t>(stream), d_y, d_pre, d_post, d_bias, act, rows,
+                           batch);
+    };
+    if (vec) go(k_bias_act<4>);
+    else go(k_bias_act<1>);
     return int(hipGetLastError());
 }
 
