@@ -471,6 +471,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
 #pragma unroll
             for (int T = 0; T < 2; ++T)
                 acc[i][T] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], b[T][kk], acc[i][T], 0, 0, 0);
+        // Q6_K's operands (6.7 VALU per MFMA) came out in runs of up to 100 between MFMAs: asked for
+        // 4 after each, 14336->4096 M = 509 runs 89.5 against 91.6 us and 4096->14336 M = 2047 272
+        // against 283. Q4_K and Q8_0 ran slower so (78.4 against 73.7 and 82.6 against 81.4 at M = 512).
+        if constexpr (std::is_same<GP, GemmQ6>::value) {
+#pragma unroll
+            for (int i = 0; i < 2 * TM; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
+            }
+        }
         __builtin_amdgcn_sched_barrier(0x6);
     };
     auto step = [&](auto E, int s) {

@@ -308,14 +308,18 @@ struct GemmQ6 {  // Q6_K: q = lo4 | hi2 << 4, w = (d/255)*u*(q - 32)
         typename GemmCodes<4>::C nib{c.c, 0u};
         uint32_t se[2][2], so[2][2];
         spread6(nib, c.h, lane, se, so);
-        const auto dt = __builtin_amdgcn_permlane32_swap(__float_as_uint(c.d), __float_as_uint(c.d), false, false);
-        const auto mt = __builtin_amdgcn_permlane32_swap(c.mw, c.mw, false, false);
+        // the own row's scales, handed to the tiles' lanes as one packed pair (as GemmKQ)
+        float w0 = wk[0], w1 = wk[1];
+        asm("" : "+v"(w0), "+v"(w1));
+        const float d255 = c.d * (((lane & 32) ? w1 : w0) * (1.0f / 255.0f));
+        const half2v scp = {_Float16(d255 * float(c.mw & 0xFFu)), _Float16(d255 * float((c.mw >> 8) & 0xFFu))};
+        const auto sc2 = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, scp),
+                                                          __builtin_bit_cast(uint32_t, scp), false, false);
 #pragma unroll
         for (int T = 0; T < 2; ++T) {
-            const float d255 = __uint_as_float(dt[T]) * (wk[T] * (1.0f / 255.0f));
-            const _Float16 sc0 = _Float16(d255 * float(mt[T] & 0xFFu)), sc1 = _Float16(d255 * float((mt[T] >> 8) & 0xFFu));
-            const _Float16 mn0 = _Float16(-32.0f) * sc0, mn1 = _Float16(-32.0f) * sc1;
-            const half2v s0 = {sc0, sc0}, s1 = {sc1, sc1}, n0 = {mn0, mn0}, n1 = {mn1, mn1};
+            const half2v k32 = {_Float16(-32.0f), _Float16(-32.0f)};
+            const half2v sp = __builtin_bit_cast(half2v, uint32_t(sc2[T])), np = sp * k32;
+            const half2v s0 = {sp.x, sp.x}, s1 = {sp.y, sp.y}, n0 = {np.x, np.x}, n1 = {np.y, np.y};
             bf[T][0] = __builtin_bit_cast(half8, dequant8s<6>(se[T][0], so[T][0], s0, n0));
             bf[T][1] = __builtin_bit_cast(half8, dequant8s<6>(se[T][1], so[T][1], s1, n1));
         }
