@@ -107,6 +107,26 @@ def test_batched_forward_route_keeps_the_result():
     d.free()
 
 
+@pytest.mark.parametrize("entry", ["wv_matvec_dev", "wv_matvec_dev_noalloc"])
+def test_batched_forward_past_the_grid_limit(entry):
+    """A batch of three rows more than one launch takes: the last part runs on the whole batch's plan, for which the
+    scratch (none) was sized, though three rows by themselves would split K."""
+    import torch
+    rows, cols, batch = 70, 2048, 65535 * 8 + 3
+    print(f"[gpu] batched past the grid limit, {entry}", flush=True)
+    p, d, rng = make("Q8_0", rows, cols, 7)
+    base = rng.standard_normal((16, cols)).astype(np.float32)
+    ref = torch.from_numpy(np.asarray(reference(p, base), np.float64)).cuda()
+    x = torch.from_numpy(base).cuda().repeat((batch + 15) // 16, 1)[:batch].contiguous()
+    y = torch.full((batch, rows), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    wv.check(getattr(wv.lib(), entry)(d.handle, x.data_ptr(), y.data_ptr(), batch, None))
+    wv.sync()
+    for i in range(16):  # row 16 k + i has x of row i
+        assert float((y[i::16].double() - ref[i]).abs().max() / ref[i].abs().max()) <= TOL
+    d.free()
+
+
 @pytest.mark.parametrize("fmt", FMTS)
 def test_batched_gradient_formats(fmt):
     rows, cols = 4700, 2304  # a ragged last row group; 9 super-blocks over the 8 XCDs; one slice of 8 waves

@@ -433,10 +433,12 @@ size_t gemv_b_scratch_floats(const DevBlob& b, int batch) {
 int launch_gemv_b(const DevBlob& b, const float* d_x, float* d_y, int batch, void* stream, float* d_scratch) {
     hipStream_t s = static_cast<hipStream_t>(stream);
     constexpr int kMaxRows = 65535 * 8;  // the grid's y limit
+    // One plan for every part of a batch past the limit, the one that the
+    // scratch was sized for: a short last part planned by itself would split K.
+    const GemvBPlan p = gemv_b_plan(b, batch);
+    if (p.splits > 1 && !d_scratch) return int(hipErrorInvalidValue);
     for (int r0 = 0; r0 < batch; r0 += kMaxRows) {
         const int nb = std::min(kMaxRows, batch - r0);
-        const GemvBPlan p = gemv_b_plan(b, nb);
-        if (p.splits > 1 && !d_scratch) return int(hipErrorInvalidValue);
         GemvBArgs ga;
         ga.w = b.rpl;
         ga.w.mode = RPL_STORE;
