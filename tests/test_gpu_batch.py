@@ -96,6 +96,24 @@ def test_batched_forward_nonfinite(fmt):
     d.free()
 
 
+@pytest.mark.parametrize("fmt", ["Q2_K", "Q3_K", "Q4_K", "Q5_K", "Q6_K", "Q8_0", "Q4_0", "IQ1_S", "IQ3_S"])
+def test_batched_forward_infinities_keep_their_sign(fmt):
+    """An infinite x gives the infinity that the weight's sign asks for, or NaN (a weight that is zero, or is a code
+    product and a min of opposite signs); never the other infinity."""
+    rows, cols = 4100, 4096
+    print(f"[gpu] batched infinities {fmt}", flush=True)
+    p, d, rng = make(fmt, rows, cols, 4)
+    x = rng.standard_normal((7, cols)).astype(np.float32)
+    x[2, 300], x[3, 4095] = np.inf, -np.inf
+    with np.errstate(invalid="ignore"):
+        ref = np.asarray(reference(p, x), np.float64)
+    y = d.matvec(x)
+    for i in (2, 3):
+        inf = np.isinf(y[i])
+        assert (inf | np.isnan(y[i])).all() and (np.sign(y[i][inf]) == np.sign(ref[i][inf])).all()
+    d.free()
+
+
 def test_batched_forward_route_keeps_the_result():
     """The same rows below and above the work at which the batched kernel takes over agree to the f32 bar."""
     rows, cols = 4099, 4096

@@ -190,10 +190,10 @@ __global__ void __launch_bounds__(64 * b_waves(NQ)) k_gemv_b(GemvBArgs ga) {
                     v[i] = make_float4(v[i].x * up, v[i].y * up, v[i].z * up, v[i].w * up);
                     if constexpr (GP::kMin) sum[i] = (v[i].x + v[i].y) + (v[i].z + v[i].w);
                 }
-                // A non-finite x takes part as itself: in the code products where the format has
-                // only those, else through the group sum alone (its planes 0). Either way it leaves
-                // no output of its row finite.
-                if (odd && GP::kMin) {
+                // A non-finite x takes part as itself, in the code products and in the group sums, and
+                // leaves no output of its row finite. With f32 mins, whose group's products and sum may
+                // be infinities of opposite signs, it does so through the sum alone, as in the one-row kernels.
+                if (odd && kVM) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i) v[i] = finite_or_0(v[i]);
                 }
