@@ -64,7 +64,7 @@ def test_batched_forward_tiles(fmt, shape):
 @pytest.mark.parametrize("fmt", ["Q4_K", "Q6_K", "Q4_1"])
 def test_batched_forward_magnitudes(fmt):
     """Each batch row and super-block has its own power of two: rows of 1e-30 and 1e30 beside ordinary
-    ones, an outlier channel (the other columns keep 2^-40 of it), an all-zero row."""
+    ones, an outlier channel (the other columns keep 2^-51 of it), an all-zero row."""
     rows, cols = 4100, 4096
     print(f"[gpu] batched magnitudes {fmt}", flush=True)
     p, d, rng = make(fmt, rows, cols, 3)
@@ -77,6 +77,24 @@ def test_batched_forward_magnitudes(fmt):
     live = [0, 1, 2, 3, 5, 6]
     assert rowwise(y[live].astype(np.float64), ref[live]) <= TOL
     assert (y[4] == 0).all()
+    d.free()
+
+
+@pytest.mark.parametrize("fmt", ["Q4_1", "Q5_1", "Q6_K", "Q8_0"])
+@pytest.mark.parametrize("mag", [1e8, -1e9])
+def test_batched_forward_dead_channel(fmt, mag):
+    """A channel of 1e8 that no weight takes up leaves the other columns' N(0, 1) at the bar: the halves hold them
+    to 2^-51 of it (1e9 gives 4.4e-7; 2^-39, without the lo half's own scale, gave 2.9e-5 and 1.9e-4)."""
+    rows, cols = 4100, 4096
+    print(f"[gpu] batched dead channel {fmt} {mag:g}", flush=True)
+    rng = np.random.default_rng(9)
+    w = (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32)
+    w[:, 64:96] = 0  # whole blocks: no min either
+    p = wv.pack(fmt, w.reshape(-1), rows, cols)
+    d = wv.upload(p)
+    x = rng.standard_normal((7, cols)).astype(np.float32)
+    x[:, 77] = mag
+    assert rowwise(d.matvec(x), reference(p, x)) <= TOL
     d.free()
 
 

@@ -11,12 +11,15 @@
 //   * the codes are the B operand of v_mfma_f32_32x32x16_f16 as they are,
 //     integers exact in fp16 (GP::codes); a 16-column step is one group of
 //     the 16-column formats, so scales stay out of the products;
-//   * each f32 x is two fp16 halves, x * 2^s = hi + lo, hi the nearest fp16
-//     and lo the nearest to the remainder (exact in f32), with 2^s taking the
-//     row's largest |x| of the super-block into [2^14, 2^15): the pair is
-//     within 2^-23 of x (about f32's own rounding), elements far below the
-//     largest within 2^-40 of it. hi and lo are different rows of the A
-//     operand, so one product gives both sums of 8 or 16 batch rows;
+//   * each f32 x is two fp16 halves, x * 2^s = hi + 2^-12 lo, hi the nearest
+//     fp16 and lo the nearest to 2^12 times the remainder (exact in f32), with
+//     2^s taking the row's largest |x| of the super-block into [2^14, 2^15):
+//     the pair is within 2^-23 of x (f32's own rounding is 2^-24) down to
+//     2^-28 of the largest and within 2^-51 of the largest below, where
+//     the one-row kernels' fixed point holds 2^-23 of a 32-column chunk's
+//     largest. Without the 2^12, lo's smallest step left 2^-39, and a dead
+//     channel of 1e8 beside N(0, 1) cost Q4_1 2.9e-5. hi and lo are different
+//     rows of the A operand, so one product gives both sums of 8 or 16 batch rows;
 //   * D holds exact products summed in f32; the group's scale meets it in f32
 //     FMAs on the VALU, 2^-s once per super-block.
 // Measured (Q4_K, us a call, one row kernel before): 4096->14336 12.9 / 15.1 /
@@ -116,8 +119,11 @@ __device__ __forceinline__ bool scale_fields(const float4 (&v)[4], uint32_t (&f)
     for (int i = 0; i < 4; ++i) f[i] = min(253u, 268u - (w[i] >> 23));
     return odd;
 }
-// x - float(h), exact where h is the fp16 nearest x
-__device__ __forceinline__ float rest(float x, _Float16 h) { return fmaf(float(h), -1.0f, x); }
+// 2^12 (x - float(h)), exact where h is the fp16 nearest x, |x| <= 2^15: at most 2^15
+constexpr float kLoScale = 4096.0f;
+__device__ __forceinline__ float rest(float x, _Float16 h) { return fmaf(float(h), -1.0f, x) * kLoScale; }
+// The sum of a product's hi and lo rows.
+__device__ __forceinline__ float hi_lo(float hi, float lo) { return fmaf(lo, 1.0f / kLoScale, hi); }
 
 // One block: 64 rows x 8 NQ batch rows x one K split, its W waves `per`
 // consecutive super-blocks each. Per super-block a wave converts its x into
@@ -282,7 +288,7 @@ __global__ void __launch_bounds__(64 * b_waves(NQ)) k_gemv_b(GemvBArgs ga) {
 #pragma unroll
                     for (int kk = 0; kk < NG; ++kk)
 #pragma unroll
-                        for (int r = 0; r < NR; ++r) s[T][r] = fmaf(d[T][kk][r] + d[T][kk][NR + r], cs[T][kk], s[T][r]);
+                        for (int r = 0; r < NR; ++r) s[T][r] = fmaf(hi_lo(d[T][kk][r], d[T][kk][NR + r]), cs[T][kk], s[T][r]);
                 if constexpr (kVM) {
 #pragma unroll
                     for (int kk = 0; kk < NG; ++kk)
@@ -324,7 +330,7 @@ __global__ void __launch_bounds__(64 * b_waves(NQ)) k_gemv_b(GemvBArgs ga) {
                     const half8 b8 = __builtin_bit_cast(half8, make_uint4(bm[T][0], bm[T][1], bm[T][2], bm[T][3]));
                     const f32x16 d = __builtin_amdgcn_mfma_f32_32x32x16_f16(sa, b8, z, 0, 0, 0);
 #pragma unroll
-                    for (int r = 0; r < NR; ++r) s[T][r] = fmaf(d[r] + d[NR + r], dm[T], s[T][r]);
+                    for (int r = 0; r < NR; ++r) s[T][r] = fmaf(hi_lo(d[r], d[NR + r]), dm[T], s[T][r]);
                 }
             }
 #pragma unroll
