@@ -300,3 +300,28 @@ def test_prefill_256_token_tiles(fmt, m, cols):
     assert normwise(y, ref) <= TOL_MFMA
     assert normwise(y[:, 7], ref[:, 7]) <= 4 * TOL_MFMA  # the tiny row on its own: fp16's precision, not subnormal
     d.free()
+
+
+@pytest.mark.parametrize("m", [32, 256])
+def test_prefill_q6k_scales_are_rounded_once(m):
+    """One-hot X reads the fp16 weights out of the GEMM (32 tokens: the register kernel, 256: the tiled one): q * sc -
+    32 * sc rounded to fp16, with sc the fp16 nearest to the exact product of d / 255 and the sub-scale, not to its f32
+    rounding (some 65536 * 5e-5 scales differ by a step)."""
+    rows, cols = 8192, 256
+    print(f"[gpu] prefill Q6_K scales M={m}", flush=True)
+    rng = np.random.default_rng(31)
+    p = wv.pack("Q6_K", (rng.standard_normal(rows * cols) * 0.02).astype(np.float32), rows, cols)
+    d = wv.upload(p)
+    y = np.zeros((cols, rows), np.float32)
+    for c in range(0, cols, m):
+        y[c:c + m] = d.matmul(np.eye(cols, dtype=np.float32)[c:c + m])
+    raw = p.raw.reshape(rows, 216)  # d, dmin (f32), 16 sub-scales, 256 6-bit codes, four to three bytes
+    dd = np.ascontiguousarray(raw[:, :4]).view(np.float32)
+    b = raw[:, 24:].reshape(rows, 64, 3).astype(np.int64)
+    q = np.stack((b[..., 0] & 63, (b[..., 0] >> 6 | b[..., 1] << 2) & 63, (b[..., 1] >> 4 | b[..., 2] << 4) & 63,
+                  b[..., 2] >> 2), 2).reshape(rows, 16, 16)
+    d255 = dd * np.float32(1.0 / 255.0)
+    sc = (d255.astype(np.float64) * np.maximum(raw[:, 8:24], 1)).astype(np.float16).astype(np.float64)
+    want = (q * sc[..., None] - 32.0 * sc[..., None]).astype(np.float16).reshape(rows, cols)
+    assert np.array_equal(y.T, want.astype(np.float32))
+    d.free()

@@ -308,13 +308,16 @@ struct GemmQ6 {  // Q6_K: q = lo4 | hi2 << 4, w = (d/255)*u*(q - 32)
         typename GemmCodes<4>::C nib{c.c, 0u};
         uint32_t se[2][2], so[2][2];
         spread6(nib, c.h, lane, se, so);
-        // the own row's scales, handed to the tiles' lanes as one packed pair (as GemmKQ)
+        // The own row's scales, handed to the tiles' lanes as one packed pair (as GemmKQ). Each is rounded once,
+        // by the instruction that multiplies: as a conversion of two f32 products the pair is rounded twice, and a
+        // block's outputs moved by 3.5e-6.
         float w0 = wk[0], w1 = wk[1];
         asm("" : "+v"(w0), "+v"(w1));
         const float d255 = c.d * (((lane & 32) ? w1 : w0) * (1.0f / 255.0f));
-        const half2v scp = {_Float16(d255 * float(c.mw & 0xFFu)), _Float16(d255 * float((c.mw >> 8) & 0xFFu))};
-        const auto sc2 = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, scp),
-                                                          __builtin_bit_cast(uint32_t, scp), false, false);
+        uint32_t scp;
+        asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(scp) : "v"(d255), "v"(float(c.mw & 0xFFu)));
+        asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(scp) : "v"(d255), "v"(float((c.mw >> 8) & 0xFFu)));
+        const auto sc2 = __builtin_amdgcn_permlane32_swap(scp, scp, false, false);
 #pragma unroll
         for (int T = 0; T < 2; ++T) {
             const half2v k32 = {_Float16(-32.0f), _Float16(-32.0f)};
