@@ -553,16 +553,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
 // so the main loop has no barrier and no LDS traffic. A step is 64 columns
 // (two chunks, four k16 MFMA steps); codes run DC steps ahead of use and X
 // fragments (L2 hits: every row group's blocks read the same X) DX steps
-// ahead, in register rings; a super-block's metadata comes in whole one
-// super-block ahead (word by word with each chunk, its 4-byte loads at a
-// 32-byte stride filled the L1: Q4_K 4096->14336 M = 32 19.5 against 21.2 us,
-// 4096->4096 17.1 against 18.2). Every weight is dequantized once per token block.
+// ahead, in register rings. A super-block's metadata comes in whole one
+// super-block ahead where GP::kMetaAhead says so (word by word with each chunk,
+// its 4-byte loads at a 32-byte stride filled the L1: Q4_K 4096->14336 M = 32
+// 19.5 against 21.2 us, 4096->4096 17.1 against 18.2), else with each chunk.
+// Every weight is dequantized once per token block.
 // The W waves' partial tiles meet in LDS after the loop and are added in wave
 // order (deterministic), one 32-token tile at a time.
 template <class GP, int TM, int DC, int DX, int NT, bool WF>
 __global__ void __launch_bounds__(NT) k_gemm_rg(GemmArgs ga, int per) {
     constexpr int BM = 32 * TM;
     static_assert(4 % DC == 0 && 4 % DX == 0, "the rings must divide the 4 steps of a super-block");
+    constexpr bool kAhead = TM <= GP::kMetaAhead;  // metadata a super-block ahead, else with each chunk
+    constexpr int DU = kAhead ? 4 : DC > DX ? DC : DX;  // loop unroll: ring positions (and metadata words) are compile-time
     extern __shared__ float red[];  // [W][2][16][64] partial tiles of one 32-token tile
     const RplArgs& a = ga.w;
     const int t = threadIdx.x, lane = t & 63, W = blockDim.x >> 6;
@@ -577,7 +580,7 @@ __global__ void __launch_bounds__(NT) k_gemm_rg(GemmArgs ga, int per) {
     if constexpr (WF) row_factors(a, g, lane, wk);
 
     struct Codes {
-        typename GP::Codes c[2];  // the step's two chunks of this lane's row
+        std::conditional_t<kAhead, typename GP::Codes, typename GP::Ch> c[2];  // the step's two chunks of this lane's row
     };
     struct Xf {
         uint4 v[TM][4];  // A fragments of the step's 4 k16 steps
@@ -585,7 +588,11 @@ __global__ void __launch_bounds__(NT) k_gemm_rg(GemmArgs ga, int per) {
     auto load_c = [&](int s, Codes& r) {
         const int64_t si = int64_t(g) * a.nsb + wsb0 + s / 4;
 #pragma unroll
-        for (int jj = 0; jj < 2; ++jj) r.c[jj] = GP::load_codes(a, rpl_chunk(a, si, 2 * (s & 3) + jj), lane);
+        for (int jj = 0; jj < 2; ++jj) {
+            const int j = 2 * (s & 3) + jj;
+            if constexpr (kAhead) r.c[jj] = GP::load_codes(a, rpl_chunk(a, si, j), lane);
+            else r.c[jj] = GP::load(a, rpl_chunk(a, si, j), si, j, lane);
+        }
     };
     auto load_m = [&](int sb) { return GP::load_meta(a, int64_t(g) * a.nsb + wsb0 + sb, lane); };
     auto load_x = [&](int s, Xf& r) {
@@ -607,18 +614,21 @@ __global__ void __launch_bounds__(NT) k_gemm_rg(GemmArgs ga, int per) {
     if (steps > 0) {
         Codes cr[DC];
         Xf xr[DX];
-        typename GP::Meta mnext = load_m(0);
+        [[maybe_unused]] typename GP::Meta mt, mnext;
+        if constexpr (kAhead) mnext = load_m(0);
 #pragma unroll
         for (int d = 0; d < (DC > DX ? DC : DX); ++d) {
             if (d < DC) load_c(min(d, steps - 1), cr[d % DC]);
             if (d < DX) load_x(min(d, steps - 1), xr[d % DX]);
             __builtin_amdgcn_sched_barrier(0);
         }
-        for (int s0 = 0; s0 < steps; s0 += 4) {  // one super-block: ring positions and metadata words are compile-time
-            const typename GP::Meta mt = mnext;
-            mnext = load_m(min(s0 + 4, steps - 4) / 4);
+        for (int s0 = 0; s0 < steps; s0 += DU) {
+            if constexpr (kAhead) {
+                mt = mnext;
+                mnext = load_m(min(s0 + 4, steps - 4) / 4);
+            }
 #pragma unroll
-            for (int d = 0; d < 4; ++d) {
+            for (int d = 0; d < DU; ++d) {
                 const int s = s0 + d;
                 const Codes cc = cr[d % DC];
                 const Xf xc = xr[d % DX];
@@ -629,7 +639,8 @@ __global__ void __launch_bounds__(NT) k_gemm_rg(GemmArgs ga, int per) {
 #pragma unroll
                 for (int jj = 0; jj < 2; ++jj) {
                     half8 bf[2][2];  // [tile][k16 step]
-                    GP::bops(GP::chunk(cc.c[jj], mt, 2 * d + jj), lane, wk, bf);
+                    if constexpr (kAhead) GP::bops(GP::chunk(cc.c[jj], mt, 2 * d + jj), lane, wk, bf);
+                    else GP::bops(cc.c[jj], lane, wk, bf);
 #pragma unroll
                     for (int kk = 0; kk < 2; ++kk)
 #pragma unroll

@@ -189,16 +189,25 @@ __device__ __forceinline__ void load_words(const RplArgs& a, int64_t si, int lan
 // of a whole super-block, loaded once for its 8 chunks (a word per chunk read
 // with every chunk costs the L1 16 lines for 256 bytes, 8 times over); Ch is
 // one chunk of both, j known at compile time, and load() a Ch read at once
-// (k_gemm_q4k_pw, whose registers hold no super-block's metadata). bops() returns the fp16 B operands bf[T][kk] of 32-row tile T and
-// k16 step kk, in X's k order [0,2,4,6,1,3,5,7], with the tile row's scales
-// and mins multiplied by its power-of-two row factor wk[T] (RplArgs::wrow)
-// before their fp16 cast.
+// (k_gemm_q4k_pw, whose registers hold no super-block's metadata). k_gemm_rg
+// takes Meta up to kMetaAhead 32-token tiles and a Ch per chunk beyond:
+// records of 16 words cost it more registers than loads (TernaryPacked
+// 4096->14336, 32 tokens, 21.1 us with Meta against 17.2, IQ3_S 64 tokens 27.0
+// against 22.9, Q5_1 128 tokens 47.4 against 43.7), and of 8 words two or more
+// tiles of the one-scale formats (BinaryPacked 14336->4096, 64 tokens, 27.9
+// against 26.8) and four of Q5_K, Q3_K and IQ4_NL (4096->14336, 128 tokens, 43.8
+// against 42.2 and 43.7 against 42.2), which load one word a chunk.
+// bops() returns the fp16 B operands bf[T][kk] of 32-row tile T and k16 step
+// kk, in X's k order [0,2,4,6,1,3,5,7], with the tile row's scales and mins
+// multiplied by its power-of-two row factor wk[T] (RplArgs::wrow) before their
+// fp16 cast.
 // For the f32-precision batched forward (k_gemv_b), codes() gives the same
 // operands as unscaled, exact fp16 code values (codes8) and scales() the f32
 // scales of rows 32T + lane % 32: one per k16 step (kTwo) or one in kk = 0 per
 // chunk, and with kMin the f32 offsets that meet the sums of x (or kMinBytes).
 template <int FB>
 struct GemmKQ {  // Q2_K, Q3_K, Q4_K, Q5_K: w = (d/255)*u*q + (dmin/127)*m
+    static constexpr int kMetaAhead = FB == 2 || FB == 4 ? 4 : 2;
     struct Ch { typename GemmCodes<FB>::C c; uint32_t mw; float2 dd; };
     using Codes = typename GemmCodes<FB>::C;
     struct Meta { uint32_t w[8]; float2 dd; };
@@ -267,6 +276,7 @@ struct GemmKQ {  // Q2_K, Q3_K, Q4_K, Q5_K: w = (d/255)*u*q + (dmin/127)*m
 };
 
 struct GemmQ6 {  // Q6_K: q = lo4 | hi2 << 4, w = (d/255)*u*(q - 32)
+    static constexpr int kMetaAhead = 4;
     struct Ch { uint4 c; uint2 h; uint32_t mw; float d; };
     struct Codes { uint4 c; uint2 h; };
     struct Meta { uint32_t w[4]; float d; };
@@ -342,6 +352,7 @@ struct GemmQ6 {  // Q6_K: q = lo4 | hi2 << 4, w = (d/255)*u*(q - 32)
 };
 
 struct GemmQ8 {  // Q8_0: w = scale*q, q int8, 32 bytes per chunk (consecutive columns)
+    static constexpr int kMetaAhead = 4;
     struct Ch { uint4 c0, c1; uint32_t sc; };
     struct Codes { uint4 c0, c1; };
     struct Meta { uint32_t w[8]; };
@@ -418,6 +429,7 @@ struct GemmQ8 {  // Q8_0: w = scale*q, q int8, 32 bytes per chunk (consecutive c
 template <int FB, bool MIN, int OFF, uint32_t XR, int GSH = 0>
 struct GemmB32 {
     static constexpr int NG = 8 >> GSH, NW = MIN ? 2 * NG : NG;
+    static constexpr int kMetaAhead = NW <= 8 ? 4 : 0;
     struct Ch { typename GemmCodes<FB>::C c; uint32_t sc, mn; };
     using Codes = typename GemmCodes<FB>::C;
     struct Meta { uint32_t w[NW]; };
@@ -504,6 +516,7 @@ template <int FB, bool SG16, int MID2, int GSH = 0>
 struct GemmLin {
     using Planes = std::conditional_t<FB == 1, GemmCodes1, GemmCodes<FB>>;
     static constexpr int NW = SG16 ? 16 : (8 >> GSH);  // metadata words per lane and super-block
+    static constexpr int kMetaAhead = NW <= 8 ? 1 : 0;
     struct Ch { typename Planes::C c; uint32_t s0, s1; };
     using Codes = typename Planes::C;
     struct Meta { uint32_t w[NW]; };
@@ -567,6 +580,7 @@ struct GemmNL {
         return uint32_t((h16(4 * n) >> sh) & 0xFF) | uint32_t((h16(4 * n + 1) >> sh) & 0xFF) << 8 |
                uint32_t((h16(4 * n + 2) >> sh) & 0xFF) << 16 | uint32_t((h16(4 * n + 3) >> sh) & 0xFF) << 24;
     }
+    static constexpr int kMetaAhead = 2;
     struct Ch { GemmCodes<4>::C c; uint32_t s0; };
     using Codes = GemmCodes<4>::C;
     struct Meta { uint32_t w[8]; };
