@@ -350,6 +350,22 @@ __global__ void __launch_bounds__(1024) k_norm_x_f16r(float* __restrict__ h, con
     }
 }
 
+// VALU instructions asked for after each MFMA of k_gemm_q4k_pw (0: the
+// compiler's own order). The builders with two code planes make 6 to 7 per
+// MFMA, which came out in runs of up to 100 between MFMAs. Measured, us, own
+// order and as set: Q6_K 14336->4096 M = 509 91.6 / 89.5; Q5_K M = 512
+// 4096->14336 96 / 84 (with 5: 91, with 9: 91), 14336->4096 100 / 96; Q3_K
+// 4096->14336 85 / 81 (with 7: 85), 14336->4096 91 / 88. Q4_K and Q8_0, with
+// fewer, ran slower with 4 (78.4 against 73.7 and 82.6 against 81.4 at M = 512).
+template <class GP>
+constexpr int kValuPerMfma = 0;
+template <>
+constexpr int kValuPerMfma<GemmQ6> = 4;
+template <>
+constexpr int kValuPerMfma<GemmKQ<5>> = 7;
+template <>
+constexpr int kValuPerMfma<GemmKQ<3>> = 9;
+
 // Each of the 4 waves owns one 64-row group of the block's 256 rows and loads
 // its row group's codes straight from the row-interleaved planes (lane l = row
 // l, 16 bytes = 32 columns per chunk). One v_permlane32_swap per code-word
@@ -471,14 +487,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
 #pragma unroll
             for (int T = 0; T < 2; ++T)
                 acc[i][T] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], b[T][kk], acc[i][T], 0, 0, 0);
-        // Q6_K's operands (6.7 VALU per MFMA) came out in runs of up to 100 between MFMAs: asked for
-        // 4 after each, 14336->4096 M = 509 runs 89.5 against 91.6 us and 4096->14336 M = 2047 272
-        // against 283. Q4_K and Q8_0 ran slower so (78.4 against 73.7 and 82.6 against 81.4 at M = 512).
-        if constexpr (std::is_same<GP, GemmQ6>::value) {
+        if constexpr (kValuPerMfma<GP> > 0) {
 #pragma unroll
             for (int i = 0; i < 2 * TM; ++i) {
                 __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
+                __builtin_amdgcn_sched_group_barrier(0x2, kValuPerMfma<GP>, 0);
             }
         }
         __builtin_amdgcn_sched_barrier(0x6);
