@@ -184,6 +184,29 @@ def test_batched_gradient_tiles(shape):
     d.free()
 
 
+@pytest.mark.parametrize("fmt", FMTS)
+def test_batched_gradient_one_pass(fmt):
+    """A shape whose batched plan fills the GPU once, which every format takes: 141 row groups over 8 waves, chains of
+    18 with a ragged end, 9 super-blocks, quartets of rows and two left over."""
+    rows, cols = 9001, 2304
+    print(f"[gpu] batched gradient, one pass, {fmt}", flush=True)
+    p, d, rng = make(fmt, rows, cols, 22)
+    check_gradient(p, d, rng, 10)
+    d.free()
+
+
+@pytest.mark.parametrize("shape", [(14337, 4096, 3), (4097, 4096, 5), (1030, 6144, 16), (500, 14336, 9), (64, 65536, 16),
+                                   (1340, 3584, 13), (2113, 7424, 6), (1985, 4864, 29)])
+def test_batched_gradient_tiles_q8(shape):
+    """Q8_0 takes the batched kernel wherever the work does: the shapes above, blocks of 3 to 7 waves (rows of 21, 34
+    and 32 groups), and a launch of 16 rows with one of 13 after it."""
+    rows, cols, batch = shape
+    print(f"[gpu] batched gradient Q8_0 {rows}x{cols} batch {batch}", flush=True)
+    p, d, rng = make("Q8_0", rows, cols, rows + batch)
+    check_gradient(p, d, rng, batch)
+    d.free()
+
+
 def check_gradient(p, d, rng, batch):
     """gx += W^T gy to the f32 bar of wv_matvec_t on each row, gx not zeroed."""
     gy = rng.standard_normal((batch, p.rows)).astype(np.float32)

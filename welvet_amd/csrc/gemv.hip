@@ -798,7 +798,7 @@ void launch_gemvt_reduce(const float* part, float* gx, int64_t cols, int nsplit,
 
 size_t matvec_t_scratch_floats(const DevBlob& b, int batch) {
     if (batch <= 0) return 0;
-    if (b.layout == LAYOUT_RPL) return rpl_t_scratch_floats(b.rpl, batch);
+    if (b.layout == LAYOUT_RPL) return rpl_t_scratch_floats(b, batch);
     if (b.layout == LAYOUT_NARROW || b.layout == LAYOUT_F32) return native_t_scratch_floats(b, batch);
     const int64_t n = std::max(raw_t_splits(b), raw_t16_slices(b));  // covers either kernel
     return size_t(n) * size_t(b.cols) * size_t(batch);

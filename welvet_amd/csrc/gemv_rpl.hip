@@ -1802,16 +1802,52 @@ RplTBPlan rpl_tb_plan(const RplArgs& a, int batch) {
     p.slices = int((a.rg_count + int64_t(p.W) * p.n - 1) / (int64_t(p.W) * p.n));
     return p;
 }
-// From 3 rows, where it runs as one slice (its chunks fill the GPU) with some
-// work, or has the work to pay for slices of a kernel this long: 4096x4096 Q6_K
-// 8 rows, one slice, 10.9 against 15.7 us; 4 rows, two slices (67 M weights x
-// rows), 11.2 against 9.4; Q4_K 14336x4096 3 rows, two slices (176 M), 23.5
-// against 32.3; one slice of 1024x14336, 4 rows (58 M) 11.9 against 10.8, 8 rows
-// 12.4 against 16.9; of 3072x7168 Q8_0, 3 rows (66 M) 11.2 against 20.0.
-bool rpl_t_batched(const RplArgs& a, int batch) {
-    const int64_t per_slice = int64_t(a.nsb) * 8 * ((batch + kRplTBatch - 1) / kRplTBatch);
+// Blocks of a plan on each CU of its busiest XCD: super-blocks go to the 8 XCDs
+// in turn, their blocks to 32 CUs.
+double rpl_t_per_cu(const RplArgs& a, int64_t blocks_per_sb) {
+    return double(((a.nsb + 7) / 8 * blocks_per_sb + 31) / 32);
+}
+// How much a row group of the batched kernel costs against one of the one-row
+// kernel: what rpl_t_batched asks the one-row plan to be longer by.
+double rpl_t_worth(int fmt) {
+    switch (fmt) {
+    case FMT_Q8_0: case FMT_IQ4_NL: return 0.0;  // always the batched one
+    case FMT_Q6_K: case FMT_Q5_1: return 1.15;
+    case FMT_Q5_K: case FMT_Q5_0: case FMT_Q4_1: return 1.47;
+    case FMT_Q4_K: return 1.6;
+    case FMT_Q3_K: case FMT_IQ3_XXS: case FMT_IQ3_S: case FMT_IQ4_XS: case FMT_AFFINE: return 1.67;
+    default: return 1.81;
+    }
+}
+// Which of the two a launch of `batch` rows takes. Both are paced by the VALU
+// of a SIMD, so a plan's length is the waves that a SIMD runs times a wave's
+// row groups (its column reductions are a quarter of a row group, or half of one
+// per 8), or one wave's latency; a second launch is 24 and 16 of those units.
+// Two waves of the batched kernel fit a SIMD (its 5- to 8-wave blocks take a CU
+// each and leave the rest of it idle), four of the one-row kernel. The batched plan rounds rows up to
+// quartets and has few, long blocks: 5 rows of 4096x14336 are two quartets
+// (Q4_K 43.9 us against 32.9 on the one-row kernel), 12 rows of 4096x4096 384
+// blocks on 256 CUs (22.4 against 18.0), where 8 rows of 14336x4096 fill them
+// once (36 against 60). The formats differ in what they pay to decode, which
+// the one-row kernel does for every row. The bounds are those at which a
+// sweep met (20 formats, 12 shapes from 1024x4096 to 32000x4096 and 260 drawn
+// ones, 3 to 16 rows), on the one-row kernel's side: of 1760 calls 21 run over
+// 2.5 % slower than on that, to 10 %, and 69 would gain as much on the other;
+// with the work alone as the rule 40 % ran slower, to 50 %. From 3 rows and, one slice, 62 M weights x rows (1024x14336 Q4_K, 4
+// rows, 58 M, 11.9 against 10.8 us), or 150 M to pay for slices (4096x4096, 4
+// rows, 67 M, 11.2 against 9.4).
+bool rpl_t_batched(const DevBlob& b, int batch) {
+    const RplArgs& a = b.rpl;
     const double work = double(batch) * double(a.rows) * double(a.nsb) * 256.0;
-    return batch >= kRplTBatch - 1 && work >= (per_slice >= kRplTMinBlocks ? 62e6 : 150e6);
+    if (batch < kRplTBatch - 1 || work < 62e6) return false;
+    const int64_t quads = (batch + kRplTBatch - 1) / kRplTBatch;
+    if (work < 150e6 && int64_t(a.nsb) * 8 * quads < kRplTMinBlocks) return false;
+    const RplTPlan o = rpl_t_plan(a, batch);
+    const RplTBPlan p = rpl_tb_plan(a, batch);
+    const double ow = o.W > 8 ? (o.W + 3) / 4 : o.W / 4.0, pw = p.W > 6 ? 2.0 : p.W > 4 ? 1.75 : p.W / 4.0;
+    const double one = std::max(1.0, rpl_t_per_cu(a, 4 * int64_t(batch) * o.slices) * ow) * (o.GP + 0.25) + (o.slices > 1 ? 24 : 0);
+    const double bat = std::max(1.5, rpl_t_per_cu(a, 8 * quads * p.slices) * pw) * (p.n + 0.5 * ((p.n + 7) / 8)) + (p.slices > 1 ? 16 : 0);
+    return one >= rpl_t_worth(b.fmt) * bat;
 }
 
 template <class P>
@@ -1820,7 +1856,7 @@ int launch_rpl_tr(const DevBlob& bl, const float* gy, float* gx, int batch, hipS
     const int64_t cols = int64_t(a.nsb) * 256;
     for (int b0 = 0; b0 < batch; b0 += kRplTMaxBatch) {
         const int nb = std::min(kRplTMaxBatch, batch - b0);
-        if (rpl_t_batched(a, nb)) {
+        if (rpl_t_batched(bl, nb)) {
             const RplTBPlan p = rpl_tb_plan(a, nb);
             if (p.slices > 1 && !part) return int(hipErrorInvalidValue);
             const dim3 grid(unsigned((a.nsb + 7) / 8 * 64), unsigned(p.slices), unsigned((nb + kRplTBatch - 1) / kRplTBatch));
@@ -2116,13 +2152,14 @@ int rpl_fuse_pairs(const DevBlob& a, const DevBlob& b, DevBlob& out, void* strea
     return int(e);
 }
 
-size_t rpl_t_scratch_floats(const RplArgs& a, int batch) {
+size_t rpl_t_scratch_floats(const DevBlob& b, int batch) {
+    const RplArgs& a = b.rpl;
     // batch rows go kRplTMaxBatch per launch (the last launch may take fewer)
     size_t most = 0;
     const int full = std::min(batch, kRplTMaxBatch), rest = batch % kRplTMaxBatch;
     for (int nb : {full, rest}) {
         if (nb <= 0) continue;
-        const int slices = rpl_t_batched(a, nb) ? rpl_tb_plan(a, nb).slices : rpl_t_plan(a, nb).slices;
+        const int slices = rpl_t_batched(b, nb) ? rpl_tb_plan(a, nb).slices : rpl_t_plan(a, nb).slices;
         if (slices > 1) most = std::max(most, size_t(slices) * size_t(nb) * size_t(a.nsb) * 256);
     }
     return most;

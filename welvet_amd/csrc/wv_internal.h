@@ -323,7 +323,7 @@ int launch_norm_x_f16r(float* h, const float* a, int a_splits, int64_t a_stride,
                        float* xscale, int M, int dim, double eps, bool frag, void* stream);
 // MatVecT on LAYOUT_RPL (slice partials in d_scratch when the plan has several slices).
 int launch_rpl_matvec_t(const DevBlob& b, const float* d_gy, float* d_gx, int batch, void* stream, float* d_scratch);
-size_t rpl_t_scratch_floats(const RplArgs& a, int batch);
+size_t rpl_t_scratch_floats(const DevBlob& b, int batch);
 // gx[b][c] += sum_k part[(b*nsplit + k)*cols + c], k ascending.
 void launch_gemvt_reduce(const float* part, float* gx, int64_t cols, int nsplit, int batch, void* stream);
 // The elementwise applyBiasAct epilogue over y[batch][rows] (layouts without a fused one).
