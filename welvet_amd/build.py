@@ -31,6 +31,7 @@ CXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-pthread", "-ffp-contract=off", "-Wa
 
 HIP_SOURCES = ["runtime.hip", "gemv.hip", "gemv_rpl.hip", "gemv_batch.hip", "gemm_rpl.hip", "decode.hip", "native.hip"]
 CXX_SOURCES = ["pack.cpp"]
+GEMM_PARTS = 8  # kGemmParts of csrc/gemm_tiles.h
 
 
 def _run(cmd):
@@ -43,8 +44,11 @@ def _run(cmd):
 
 def build(verbose: bool = False) -> str:
     os.makedirs(OBJ, exist_ok=True)
-    jobs = [[HIPCC, *HIP_FLAGS, "-c", os.path.join(CSRC, src), "-o", os.path.join(OBJ, src + ".o")]
-            for src in HIP_SOURCES]
+    # the slowest first
+    jobs = [[HIPCC, *HIP_FLAGS, f"-DWV_GEMM_PART={i}", "-c", os.path.join(CSRC, "gemm_tiles.hip"),
+             "-o", os.path.join(OBJ, f"gemm_tiles.hip.{i}.o")] for i in range(GEMM_PARTS)]
+    jobs += [[HIPCC, *HIP_FLAGS, "-c", os.path.join(CSRC, src), "-o", os.path.join(OBJ, src + ".o")]
+             for src in HIP_SOURCES]
     jobs += [["g++", *CXX_FLAGS, "-c", os.path.join(CSRC, src), "-o", os.path.join(OBJ, src + ".o")]
              for src in CXX_SOURCES]
     workers = max(1, min(len(jobs), int(os.environ.get("MAX_JOBS", "0")) or (os.cpu_count() or 1)))

@@ -629,6 +629,24 @@ struct GemmNL {
     }
 };
 
+// The part of gemm_tiles.hip (gemm_tiles.h) that compiles a builder's kernels:
+// two for each builder that takes longest (the second for its 256-token tiles),
+// one for the linear codes and one for the rest.
+template <class GP>
+struct GemmPart : std::integral_constant<int, 7> {};
+template <>
+struct GemmPart<GemmKQ<3>> : std::integral_constant<int, 0> {};
+template <>
+struct GemmPart<GemmKQ<5>> : std::integral_constant<int, 2> {};
+template <>
+struct GemmPart<GemmQ6> : std::integral_constant<int, 4> {};
+template <int FB, bool SG16, int MID2, int GSH>
+struct GemmPart<GemmLin<FB, SG16, MID2, GSH>> : std::integral_constant<int, 6> {};
+template <class GP>
+constexpr int gemm_part(bool tall) {
+    return GemmPart<GP>::value + (tall && GemmPart<GP>::value < 6 ? 1 : 0);
+}
+
 // Calls go.template run<GP>() with the B-operand builder of b's format.
 template <class Go>
 int with_builder(const DevBlob& b, const Go& go) {
