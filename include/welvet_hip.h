@@ -199,13 +199,22 @@ int wv_weight_bytes(uint64_t *resident, uint64_t *budget);
  * (simd.go:201-214): f32 weights, f64 sums. */
 int wv_matvec(uint64_t handle, const float *x, float *y, int32_t batch);
 
-/* Device-pointer form of wv_matvec, enqueued on `stream`. */
+/* Device-pointer form of wv_matvec, enqueued on `stream`. Batches of about 10^8
+ * weights x rows and more run on kernels that decode each weight once for 8 or
+ * 16 rows. Products that split K (or, of a gradient, the rows) keep partials in
+ * device scratch that the library holds and shares between calls in stream
+ * order. While `stream` is captured into a HIP graph, a batch whose one-row
+ * kernels need no scratch runs on those, so that the graph holds plain launches
+ * (so also wv_dense_forward_dev and wv_matvec_t_dev); products that need it in
+ * either form, and the block products, belong into a graph only through
+ * wv_matvec_dev_noalloc. */
 int wv_matvec_dev(uint64_t handle, const float *d_x, float *d_y, int32_t batch, void *stream);
 
 /* wv_matvec_dev that allocates nothing. It has no counterpart in the
  * reference: it is for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
- * Kernels that need scratch (the K-split partials of large-K shapes) use one
+ * Kernels that need scratch (the partials of K splits: large-K shapes, and
+ * batches whose rows alone would leave the GPU idle) use one
  * fixed 4 MiB device array per GPU, held until the process ends, instead of a
  * per-call allocation; a shape whose partials (up to 8 batch rows x the K
  * split x the rows padded to 64) exceed 2^20 floats fails with WV_E_SHAPE

@@ -163,6 +163,50 @@ def test_batched_forward_past_the_grid_limit(entry):
     d.free()
 
 
+@pytest.mark.parametrize("case", [("wv_dense_forward_dev", "Q4_K", 4096, 4096, 8), ("wv_matvec_dev", "Q8_0", 4096, 4096, 5),
+                                  ("wv_matvec_t_dev", "Q8_0", 8000, 5120, 4)])
+def test_batches_under_capture_record_plain_launches(case):
+    """Under a caller's capture a batch whose one-row kernels need no scratch takes none, though its batched kernel
+    splits K (or the rows, of a gradient): each replay gives the one-row kernels' result (a forward row's bits are
+    those it has alone), with eager work that does use the scratch between."""
+    import torch
+    entry, fmt, rows, cols, batch = case
+    print(f"[gpu] captured {case}", flush=True)
+    p, d, rng = make(fmt, rows, cols, 8)
+    L, t = wv.lib(), entry == "wv_matvec_t_dev"
+    nin, nout = (rows, cols) if t else (cols, rows)
+    x = torch.from_numpy(rng.standard_normal((batch, nin)).astype(np.float32)).cuda()
+    y, alone, eager = (torch.zeros((batch, nout), device="cuda") for _ in range(3))
+
+    def call(xp, yp, b, s):
+        if entry == "wv_dense_forward_dev":
+            wv.check(L.wv_dense_forward_dev(d.handle, xp, yp, None, b, None, wv.ACT["linear"], s))
+        else:
+            wv.check(getattr(L, entry)(d.handle, xp, yp, b, s))
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        for i in range(batch):
+            call(x[i].data_ptr(), alone[i].data_ptr(), 1, s.cuda_stream)
+    s.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        call(x.data_ptr(), y.data_ptr(), batch, s.cuda_stream)
+    for _ in range(3):
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert rowwise(y.cpu().numpy().astype(np.float64), alone.cpu().numpy()) <= TOL
+        assert t or torch.equal(y, alone)
+        eager.zero_()
+        torch.cuda.synchronize()
+        call(x.data_ptr(), eager.data_ptr(), batch, s.cuda_stream)
+        s.synchronize()
+        assert not torch.equal(eager, y)  # the batched kernel's sums, in another order
+        assert rowwise(eager.cpu().numpy().astype(np.float64), alone.cpu().numpy()) <= TOL
+    d.free()
+
+
 @pytest.mark.parametrize("fmt", FMTS)
 def test_batched_gradient_formats(fmt):
     rows, cols = 4700, 2304  # a ragged last row group; 9 super-blocks over the 8 XCDs; one slice of 8 waves

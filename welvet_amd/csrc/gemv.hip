@@ -749,7 +749,9 @@ RawTFn pick_raw_t(int fmt) {
 
 }  // namespace
 
-size_t matvec_scratch_floats(const DevBlob& b, int batch) { return rpl_scratch_floats(b, batch); }
+size_t matvec_scratch_floats(const DevBlob& b, int batch, bool one_row) {
+    return one_row ? rpl_rowwise_scratch_floats(b, batch) : rpl_scratch_floats(b, batch);
+}
 
 int launch_matvec(const DevBlob& b, const float* d_x, float* d_y, int batch, void* stream, float* d_scratch,
                   const BiasAct* ba) {
@@ -796,9 +798,9 @@ void launch_gemvt_reduce(const float* part, float* gx, int64_t cols, int nsplit,
                        static_cast<hipStream_t>(stream), part, gx, cols, nsplit);
 }
 
-size_t matvec_t_scratch_floats(const DevBlob& b, int batch) {
+size_t matvec_t_scratch_floats(const DevBlob& b, int batch, bool one_row) {
     if (batch <= 0) return 0;
-    if (b.layout == LAYOUT_RPL) return rpl_t_scratch_floats(b, batch);
+    if (b.layout == LAYOUT_RPL) return rpl_t_scratch_floats(b, batch, one_row);
     if (b.layout == LAYOUT_NARROW || b.layout == LAYOUT_F32) return native_t_scratch_floats(b, batch);
     const int64_t n = std::max(raw_t_splits(b), raw_t16_slices(b));  // covers either kernel
     return size_t(n) * size_t(b.cols) * size_t(batch);

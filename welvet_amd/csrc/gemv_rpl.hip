@@ -1856,9 +1856,9 @@ int launch_rpl_tr(const DevBlob& bl, const float* gy, float* gx, int batch, hipS
     const int64_t cols = int64_t(a.nsb) * 256;
     for (int b0 = 0; b0 < batch; b0 += kRplTMaxBatch) {
         const int nb = std::min(kRplTMaxBatch, batch - b0);
-        if (rpl_t_batched(bl, nb)) {
+        // without scratch the one-row kernel takes what it can run without
+        if (rpl_t_batched(bl, nb) && (part || rpl_tb_plan(a, nb).slices == 1)) {
             const RplTBPlan p = rpl_tb_plan(a, nb);
-            if (p.slices > 1 && !part) return int(hipErrorInvalidValue);
             const dim3 grid(unsigned((a.nsb + 7) / 8 * 64), unsigned(p.slices), unsigned((nb + kRplTBatch - 1) / kRplTBatch));
             hipLaunchKernelGGL((k_gemvt_rpl_b<P, kRplTBatch>), grid, dim3(unsigned(64 * p.W)), 0, s, a,
                                gy + int64_t(b0) * a.rows, gx + int64_t(b0) * cols, part, nb, p.n);
@@ -1937,7 +1937,9 @@ void launch_rpl_ksum(const RplArgs& a, float* y, int batch, void* stream) {
 
 int launch_rpl(const DevBlob& b, const float* d_x, float* d_y, int batch, void* stream, int mode, const float* aux,
                float* d_scratch) {
-    if (mode == RPL_STORE && gemv_b_supported(b, batch)) return launch_gemv_b(b, d_x, d_y, batch, stream, d_scratch);
+    // without scratch the one-row kernels take a product that they can run without
+    if (mode == RPL_STORE && gemv_b_supported(b, batch) && (d_scratch || gemv_b_scratch_floats(b, batch) == 0))
+        return launch_gemv_b(b, d_x, d_y, batch, stream, d_scratch);
     RplExtra ex;
     ex.mode = mode;
     ex.aux = aux;
@@ -2152,14 +2154,14 @@ int rpl_fuse_pairs(const DevBlob& a, const DevBlob& b, DevBlob& out, void* strea
     return int(e);
 }
 
-size_t rpl_t_scratch_floats(const DevBlob& b, int batch) {
+size_t rpl_t_scratch_floats(const DevBlob& b, int batch, bool one_row) {
     const RplArgs& a = b.rpl;
     // batch rows go kRplTMaxBatch per launch (the last launch may take fewer)
     size_t most = 0;
     const int full = std::min(batch, kRplTMaxBatch), rest = batch % kRplTMaxBatch;
     for (int nb : {full, rest}) {
         if (nb <= 0) continue;
-        const int slices = rpl_t_batched(b, nb) ? rpl_tb_plan(a, nb).slices : rpl_t_plan(a, nb).slices;
+        const int slices = !one_row && rpl_t_batched(b, nb) ? rpl_tb_plan(a, nb).slices : rpl_t_plan(a, nb).slices;
         if (slices > 1) most = std::max(most, size_t(slices) * size_t(nb) * size_t(a.nsb) * 256);
     }
     return most;

@@ -218,6 +218,20 @@ struct CallScratch {
     }
 };
 
+// Floats of scratch for a product on st: `most` for its fastest kernels, and
+// none while st records a graph whose product can do without (one_row == 0):
+// the graph then holds plain launches, and nothing that it writes on a replay
+// belongs to a slot that another call may hold. 8 rows of Q4_K 14336->4096 take
+// 67 us so, 17 with the scratch of wv_matvec_dev_noalloc.
+size_t call_floats(size_t most, size_t one_row, hipStream_t st) {
+    if (!most || one_row) return most;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone ? 0 : most;
+}
+size_t fwd_floats(const DevBlob& b, int batch, hipStream_t st) {
+    return call_floats(matvec_scratch_floats(b, batch), matvec_scratch_floats(b, batch, true), st);
+}
+
 // Bounce slots of the host entry points: a pinned host buffer and a device
 // buffer of kStageBytes each, at most kStageSlots per device, made on first
 // use, held by one call at a time and kept for the process. A call that finds
@@ -1082,7 +1096,7 @@ int wv_matvec_dev(uint64_t handle, const float* d_x, float* d_y, int32_t batch, 
     (void)hipSetDevice(b.device);
     hipStream_t s = stream_or_default(stream, b.device);
     CallScratch sc;
-    int rc = sc.get(matvec_scratch_floats(b, batch), s, "MatVec: scratch");
+    int rc = sc.get(fwd_floats(b, batch, s), s, "MatVec: scratch");
     if (rc) return rc;
     const int e = launch_matvec(b, d_x, d_y, batch, s, sc.f());
     if (e != hipSuccess) return hip_fail(hipError_t(e), "MatVec: kernel launch");
@@ -1160,7 +1174,8 @@ int wv_matvec_t_dev(uint64_t handle, const float* d_gy, float* d_gx, int32_t bat
     (void)hipSetDevice(b.device);
     hipStream_t s = stream_or_default(stream, b.device);
     CallScratch sc;
-    int rc = sc.get(matvec_t_scratch_floats(b, batch), s, "MatVecT: scratch");
+    int rc = sc.get(call_floats(matvec_t_scratch_floats(b, batch), matvec_t_scratch_floats(b, batch, true), s), s,
+                    "MatVecT: scratch");
     if (rc) return rc;
     const int k = launch_matvec_t(b, d_gy, d_gx, batch, s, sc.f());
     if (k != hipSuccess) return hip_fail(hipError_t(k), "MatVecT: kernel launch");
@@ -1177,7 +1192,7 @@ int wv_matmul_dev(uint64_t handle, const float* d_x, float* d_y, int32_t m, void
     hipStream_t s = stream_or_default(stream, b.device);
     const bool gemm = gemm_supported(b, m);
     CallScratch sc;
-    int rc = sc.get(gemm ? gemm_scratch_floats(b, m) : matvec_scratch_floats(b, m), s, "MatMul: scratch");
+    int rc = sc.get(gemm ? gemm_scratch_floats(b, m) : fwd_floats(b, m, s), s, "MatMul: scratch");
     if (rc) return rc;
     const int k = gemm ? launch_gemm(b, d_x, d_y, m, s, sc.f()) : launch_matvec(b, d_x, d_y, m, s, sc.f());
     if (k != hipSuccess) return hip_fail(hipError_t(k), "MatMul: kernel launch");
@@ -1281,7 +1296,7 @@ int wv_dense_forward_dev(uint64_t handle, const float* d_x, float* d_pre, float*
     (void)hipSetDevice(b.device);
     hipStream_t s = stream_or_default(stream, b.device);
     CallScratch sc;
-    int rc = sc.get(matvec_scratch_floats(b, batch), s, "dense: scratch");
+    int rc = sc.get(fwd_floats(b, batch, s), s, "dense: scratch");
     if (rc) return rc;
     BiasAct ba;
     ba.bias = d_bias;

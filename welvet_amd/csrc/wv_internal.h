@@ -260,7 +260,8 @@ struct DevBlob {
 // Kernel launchers (gemv.hip, gemv_rpl.hip, native.hip). Return a hipError_t
 // as int. A launcher whose kernels need scratch takes it as `d_scratch` and
 // returns hipErrorInvalidValue when it is null; *_scratch_floats() give the
-// floats it needs (0: none).
+// floats it needs (0: none). A batch whose one-row kernels need none (one_row)
+// runs on those when d_scratch is null.
 int launch_rpl(const DevBlob& b, const float* d_x, float* d_y, int batch, void* stream, int mode = RPL_STORE,
                const float* aux = nullptr, float* d_scratch = nullptr);
 int launch_rpl_ex(const DevBlob& b, const float* d_x, float* d_y, int batch, void* stream, const RplExtra& ex);
@@ -275,10 +276,10 @@ void launch_rpl_ksum(const RplArgs& a, float* y, int batch, void* stream);
 bool gemv_b_supported(const DevBlob& b, int batch);
 size_t gemv_b_scratch_floats(const DevBlob& b, int batch);
 int launch_gemv_b(const DevBlob& b, const float* d_x, float* d_y, int batch, void* stream, float* d_scratch);
-size_t matvec_scratch_floats(const DevBlob& b, int batch);
+size_t matvec_scratch_floats(const DevBlob& b, int batch, bool one_row = false);
 int launch_matvec(const DevBlob& b, const float* d_x, float* d_y, int batch, void* stream, float* d_scratch,
                   const BiasAct* ba = nullptr);
-size_t matvec_t_scratch_floats(const DevBlob& b, int batch);
+size_t matvec_t_scratch_floats(const DevBlob& b, int batch, bool one_row = false);
 int launch_matvec_t(const DevBlob& b, const float* d_gy, float* d_gx, int batch, void* stream, float* d_scratch);
 // Fused row-interleaved images (gemv_rpl.hip), built on the device from
 // resident blobs of one format and width: rpl_fuse_rows stacks the parts'
@@ -323,7 +324,7 @@ int launch_norm_x_f16r(float* h, const float* a, int a_splits, int64_t a_stride,
                        float* xscale, int M, int dim, double eps, bool frag, void* stream);
 // MatVecT on LAYOUT_RPL (slice partials in d_scratch when the plan has several slices).
 int launch_rpl_matvec_t(const DevBlob& b, const float* d_gy, float* d_gx, int batch, void* stream, float* d_scratch);
-size_t rpl_t_scratch_floats(const DevBlob& b, int batch);
+size_t rpl_t_scratch_floats(const DevBlob& b, int batch, bool one_row = false);
 // gx[b][c] += sum_k part[(b*nsplit + k)*cols + c], k ascending.
 void launch_gemvt_reduce(const float* part, float* gx, int64_t cols, int nsplit, int batch, void* stream);
 // The elementwise applyBiasAct epilogue over y[batch][rows] (layouts without a fused one).
