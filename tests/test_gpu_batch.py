@@ -143,6 +143,21 @@ def test_batched_forward_route_keeps_the_result():
     d.free()
 
 
+@pytest.mark.parametrize("case", [("Q4_K", 20555, 2560, 2, False), ("Q2_K", 17087, 2304, 3, False),
+                                  ("Q4_K", 4096, 14336, 2, True), ("IQ3_S", 17087, 2560, 3, True)])
+def test_two_and_three_rows_take_the_shorter_plan(case):
+    """Past the work at which larger batches take the batched kernel, 2 and 3 rows take it where its passes over the
+    GPU are fewer or shorter: told by the bits, which a row has alone on the one-row kernel only."""
+    fmt, rows, cols, batch, batched = case
+    print(f"[gpu] route {case}", flush=True)
+    p, d, rng = make(fmt, rows, cols, 12)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    y, alone = d.matvec(x), np.concatenate([d.matvec(x[i:i + 1]) for i in range(batch)])
+    assert rowwise(y.astype(np.float64), alone) <= TOL
+    assert np.array_equal(y, alone) == (not batched)
+    d.free()
+
+
 @pytest.mark.parametrize("entry", ["wv_matvec_dev", "wv_matvec_dev_noalloc"])
 def test_batched_forward_past_the_grid_limit(entry):
     """A batch of three rows more than one launch takes: the last part runs on the whole batch's plan, for which the

@@ -73,9 +73,7 @@ struct GemvBLds {
     static constexpr int kInv = kSum + 2 * kRow, kWave = kInv + 8 * NQ;
     static_assert(16 * 8 * NQ <= 2 * kRow && kWave % 4 == 0, "group sums");
 };
-// Waves per block: one octet of batch rows leaves 128 registers a wave room
-// for 16 waves (4 per SIMD), two take 256 and 8 waves.
-constexpr int b_waves(int) { return 8; }
+constexpr int kBWaves = 8;  // per block at most: two of 256 registers on each SIMD
 
 constexpr uint32_t kInfBits = 0x7F800000u;
 __device__ __forceinline__ uint32_t abs_bits(float f) { return __float_as_uint(f) & 0x7FFFFFFFu; }
@@ -134,7 +132,7 @@ __device__ __forceinline__ float hi_lo(float hi, float lo) { return fmaf(lo, 1.0
 // 4 NQ + r add up to batch row 8(r / 4) + 4(l / 32) + r % 4 of weight row 32T
 // + l % 32. The waves' sums meet in LDS in wave order.
 template <class GP, int NQ>
-__global__ void __launch_bounds__(64 * b_waves(NQ)) k_gemv_b(GemvBArgs ga) {
+__global__ void __launch_bounds__(64 * kBWaves) k_gemv_b(GemvBArgs ga) {
     using L = GemvBLds<NQ>;
     constexpr int NT = 8 * NQ, NR = 4 * NQ, D = 4;  // D chunks of codes in flight
     constexpr int GW = GP::kTwo ? 16 : 32;  // columns per scale
@@ -394,7 +392,7 @@ GemvBPlan gemv_b_plan(const DevBlob& b, int batch) {
     const int want = int(std::max<int64_t>(1, std::min<int64_t>(kBCUs / blocks, a.nsb / 4)));
     p.sb_per_split = (a.nsb + want - 1) / want;
     p.splits = (a.nsb + p.sb_per_split - 1) / p.sb_per_split;
-    p.per = (p.sb_per_split + b_waves(p.nq) - 1) / b_waves(p.nq);
+    p.per = (p.sb_per_split + kBWaves - 1) / kBWaves;
     p.W = (p.sb_per_split + p.per - 1) / p.per;
     return p;
 }
@@ -425,10 +423,34 @@ struct GemvBGo {
 // 11.4 at 126 M; Q6_K and Q4_0 alike; Q8_0 8 rows and fewer 13.3 against 12.1
 // at 44 M, 15.4 against 10.0 at 67 M, more rows 10.9 against 11.8 at 67 M, 14.1
 // against 10.4 at 94 M. IQ4_NL's float grid is not exact in fp16.
+// Two and three rows leave most of an octet's work unused, so there the two
+// plans' times are compared (Q8_0 apart, which gains everywhere): a pass of the
+// batched kernel over the GPU takes 5 us and 6 for each super-block of a wave,
+// a K split 2 more, the one-row kernel what gemv_b_row_us says. Q4_K 2 rows:
+// 20555x2560, two passes, 22.0 us against the one-row kernel's 12.7;
+// 44096x1536 22.8 against 15.7; 4096x14336 16.3 against 18.2. Of 705 calls
+// (19 formats, 37 shapes) 11 run over 2.5 % slower than on the one-row kernel, to
+// 10 %, and 40 would gain as much here; with the lines above alone 205 ran
+// slower, to 43 %.
+static double gemv_b_row_us(int fmt) {  // us per million weights and row
+    switch (fmt) {
+    case FMT_Q2_K: return 0.105;
+    case FMT_Q6_K: case FMT_Q4_0: case FMT_Q5_0: return 0.165;
+    case FMT_IQ2_XS: case FMT_IQ3_S: case FMT_IQ4_XS: case FMT_TERNARY: return 0.17;
+    case FMT_Q4_1: case FMT_Q5_1: return 0.185;
+    default: return 0.13;
+    }
+}
 bool gemv_b_supported(const DevBlob& b, int batch) {
+    if (batch < 2 || b.layout != LAYOUT_RPL || b.fmt == FMT_IQ4_NL) return false;
     const double work = double(batch) * double(b.rows) * double(b.cols);
-    const double line = b.fmt != FMT_Q8_0 ? 105e6 : batch <= 8 ? 60e6 : 90e6;
-    return batch >= 2 && b.layout == LAYOUT_RPL && b.fmt != FMT_IQ4_NL && work >= line;
+    if (work < (b.fmt != FMT_Q8_0 ? 105e6 : batch <= 8 ? 60e6 : 90e6)) return false;
+    if (batch > 3 || b.fmt == FMT_Q8_0) return true;
+    const GemvBPlan p = gemv_b_plan(b, batch);
+    // blocks of up to 4 waves run two to a CU
+    const int64_t blocks = int64_t(b.rpl.rg_count) * p.splits, fit = p.W <= 4 ? 2 * kBCUs : kBCUs;
+    const double passes = double((blocks + fit - 1) / fit);
+    return 6.0 + gemv_b_row_us(b.fmt) * work * 1e-6 >= passes * (5.0 + 6.0 * p.per) + (p.splits > 1 ? 2.0 : 0.0);
 }
 
 size_t gemv_b_scratch_floats(const DevBlob& b, int batch) {
