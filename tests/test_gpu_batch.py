@@ -144,7 +144,7 @@ def test_batched_forward_route_keeps_the_result():
 
 
 @pytest.mark.parametrize("case", [("Q4_K", 20555, 2560, 2, False), ("Q2_K", 17087, 2304, 3, False),
-                                  ("Q4_K", 4096, 14336, 2, True), ("IQ3_S", 17087, 2560, 3, True)])
+                                  ("Q4_K", 4096, 14336, 2, True), ("IQ3_S", 10465, 4096, 3, True)])
 def test_two_and_three_rows_take_the_shorter_plan(case):
     """Past the work at which larger batches take the batched kernel, 2 and 3 rows take it where its passes over the
     GPU are fewer or shorter: told by the bits, which a row has alone on the one-row kernel only."""
