@@ -344,3 +344,28 @@ def test_bias_act_large_blocks(rows, act):
     assert np.array_equal(pre, np.asarray(want_pre, np.float32).reshape(pre.shape))
     assert normwise(post, want_post) <= 1.2e-7  # one ulp of f32 (2^-23): the device's exp and tanh may round the other way
     d.free()
+
+
+@pytest.mark.parametrize("rows,batch,off", [(1024, 9000, 0), (1024, 1100, 1), (1024, 1100, 4), (12, 90000, 0), (132, 8200, 0),
+                                            (2052, 600, 0), (10, 1, 0), (33, 300, 0), (3, 70000, 1)])
+def test_bias_act_narrow_tall_and_misaligned(rows, batch, off):
+    """The epilogue where a thread takes a second group of batch rows, on layers narrower than a block, with a ragged
+    last group, and with pre and post at `off` floats past 16-byte alignment: exact, and no float outside is written."""
+    import torch
+    p, d, rng = make("Q8_0", rows, 256, rows + batch)
+    x = torch.from_numpy(rng.standard_normal((batch, 256)).astype(np.float32)).cuda()
+    bias = torch.from_numpy(rng.standard_normal(rows)).cuda()
+    n = rows * batch
+    y = torch.empty(n, device="cuda")
+    pre, post = (torch.full((n + 8,), -7.0, device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    L = wv.lib()
+    wv.check(L.wv_matvec_dev(d.handle, x.data_ptr(), y.data_ptr(), batch, None))
+    wv.check(L.wv_dense_forward_dev(d.handle, x.data_ptr(), pre.data_ptr() + 4 * off, post.data_ptr() + 4 * off, batch,
+                                    bias.data_ptr(), wv.ACT["relu"], None))
+    wv.sync()
+    want = (y.view(batch, rows).double() + bias).float().view(-1)
+    assert torch.equal(pre[off:off + n], want) and torch.equal(post[off:off + n], want.clamp(min=0))
+    for t in (pre, post):
+        assert (t[:off] == -7).all() and (t[off + n:] == -7).all()
+    d.free()

@@ -566,40 +566,48 @@ __global__ void __launch_bounds__(64) k_gemvt_reduce(const float* __restrict__ p
 // f32(y + bias) written to `pre`, post = f32(act(f64(pre))) to `post`. y and
 // pre may be the same buffer (in place; each thread reads its element before
 // writing it), so neither is declared __restrict__.
-// A thread owns V consecutive columns (V = 4: whole float4s) of every
-// gridDim.y-th batch row, its bias in registers. With one element per thread
-// and its column taken from a flat 64-bit index the division cost as much as
-// the activation: 2047 x 14336 with bias and SiLU 89 us, now 71, for 352 MB
-// (68 us at a large copy's 5.2 TB/s).
-template <int V>
+//
+// k_bias_act takes any rows and buffers, an element a thread in the order of
+// memory: blocks that each held whole columns cut the cache lines that two of
+// them write (the pass alone, 33 outputs of 30000 rows 7 to 18 us, here 5; 257
+// of 8192 11 to 14, here 8). Its division is of 32 bits wherever the elements
+// are fewer than 2^32.
+template <class U>
 __global__ void __launch_bounds__(256) k_bias_act(const float* y, float* pre, float* __restrict__ post,
-                                                  const double* __restrict__ bias, int act, int64_t rows, int batch) {
-    const int64_t c = (int64_t(blockIdx.x) * 256 + threadIdx.x) * V;
-    if (c >= rows) return;
-    double bv[V];
+                                                  const double* __restrict__ bias, int act, U rows, U n) {
+    const U i = U(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= n) return;
+    float v = y[i];
+    if (bias) v = float(double(v) + bias[i % rows]);
+    pre[i] = v;
+    post[i] = act == ACT_LINEAR ? v : float(activate_f64(double(v), act));
+}
+
+// k_bias_act4: a thread owns a float4 of columns of every gridDim.y-th group of
+// batch rows, its biases in registers; a block is nc threads of columns by `per`
+// batch rows (launch_bias_act). Where an element a thread and a 64-bit division
+// took 89 us for 2047 x 14336 with bias and SiLU, this takes 71, for 352 MB
+// (68 us at a large copy's 5.2 TB/s).
+__global__ void __launch_bounds__(512) k_bias_act4(const float4* y, float4* pre, float4* __restrict__ post,
+                                                   const double* __restrict__ bias, int act, int64_t row4s, int batch,
+                                                   int nc, int per) {
+    const int r = int(threadIdx.x) / nc;
+    const int64_t c = int64_t(blockIdx.x) * nc + (int(threadIdx.x) - r * nc);
+    if (r >= per || c >= row4s) return;
+    double bv[4];
 #pragma unroll
-    for (int k = 0; k < V; ++k) bv[k] = bias ? bias[c + k] : 0.0;
-    for (int b = blockIdx.y; b < batch; b += gridDim.y) {
-        const int64_t i = int64_t(b) * rows + c;
-        float v[V], o[V];
-        if constexpr (V == 4) {
-            const float4 t = *reinterpret_cast<const float4*>(y + i);
-            v[0] = t.x, v[1] = t.y, v[2] = t.z, v[3] = t.w;
-        } else {
-            v[0] = y[i];
-        }
+    for (int k = 0; k < 4; ++k) bv[k] = bias ? bias[4 * c + k] : 0.0;
+    for (int64_t b = int64_t(blockIdx.y) * per + r; b < batch; b += int64_t(gridDim.y) * per) {
+        const int64_t i = b * row4s + c;
+        const float4 t = y[i];
+        float v[4] = {t.x, t.y, t.z, t.w}, o[4];
 #pragma unroll
-        for (int k = 0; k < V; ++k) {
+        for (int k = 0; k < 4; ++k) {
             if (bias) v[k] = float(double(v[k]) + bv[k]);
             o[k] = act == ACT_LINEAR ? v[k] : float(activate_f64(double(v[k]), act));
         }
-        if constexpr (V == 4) {
-            *reinterpret_cast<float4*>(pre + i) = make_float4(v[0], v[1], v[2], v[3]);
-            *reinterpret_cast<float4*>(post + i) = make_float4(o[0], o[1], o[2], o[3]);
-        } else {
-            pre[i] = v[0];
-            post[i] = o[0];
-        }
+        pre[i] = make_float4(v[0], v[1], v[2], v[3]);
+        post[i] = make_float4(o[0], o[1], o[2], o[3]);
     }
 }
 
@@ -777,19 +785,32 @@ int launch_matvec(const DevBlob& b, const float* d_x, float* d_y, int batch, voi
 
 int launch_bias_act(const float* d_y, float* d_pre, float* d_post, const double* d_bias, int act, int64_t rows,
                     int batch, void* stream) {
-    if (rows * int64_t(batch) == 0) return 0;
+    const int64_t n = rows * int64_t(batch);
+    if (n == 0) return 0;
+    hipStream_t s = static_cast<hipStream_t>(stream);
     // float4s where the rows and buffers allow it and there are enough of them to fill the GPU
     auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    const bool vec = rows % 4 == 0 && aligned(d_y) && aligned(d_pre) && aligned(d_post) &&
-                     rows * int64_t(batch) >= int64_t(1) << 20;
-    const int64_t gx = (rows / (vec ? 4 : 1) + 255) / 256;
-    const dim3 grid(unsigned(gx), unsigned(std::min<int64_t>(batch, vec ? std::max<int64_t>(1, 8192 / gx) : 65535)));
-    auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, grid, dim3(256), 0, static_cast<hipStream_t>(stream), d_y, d_pre, d_post, d_bias, act, rows,
-                           batch);
-    };
-    if (vec) go(k_bias_act<4>);
-    else go(k_bias_act<1>);
+    if (rows % 4 == 0 && aligned(d_y) && aligned(d_pre) && aligned(d_post) && n >= int64_t(1) << 20) {
+        // A block is whole batch rows of a narrow layer, as many as 256 threads hold (or one more,
+        // where that leaves fewer threads of its last wave idle), else an equal share of one row.
+        const int64_t row4s = rows / 4, gx = (row4s + 511) / 512;
+        const int nc = int((row4s + gx - 1) / gx);
+        auto fill = [&](int per) { return double(per * nc) / ((per * nc + 63) / 64 * 64); };
+        int per = std::max(1, 256 / nc);
+        if (nc < 256 && fill(per + 1) > fill(per)) ++per;
+        const unsigned threads = unsigned((per * nc + 63) / 64 * 64);
+        const int64_t gy = (int64_t(batch) + per - 1) / per, most = std::max<int64_t>(1, (int64_t(1) << 21) / (gx * threads));
+        hipLaunchKernelGGL(k_bias_act4, dim3(unsigned(gx), unsigned(std::min(gy, most))), dim3(threads), 0, s,
+                           reinterpret_cast<const float4*>(d_y), reinterpret_cast<float4*>(d_pre),
+                           reinterpret_cast<float4*>(d_post), d_bias, act, row4s, batch, nc, per);
+        return int(hipGetLastError());
+    }
+    const dim3 grid(unsigned((n + 255) / 256));
+    if (n <= int64_t(UINT32_MAX) - 255)
+        hipLaunchKernelGGL(k_bias_act<uint32_t>, grid, dim3(256), 0, s, d_y, d_pre, d_post, d_bias, act, uint32_t(rows),
+                           uint32_t(n));
+    else
+        hipLaunchKernelGGL(k_bias_act<int64_t>, grid, dim3(256), 0, s, d_y, d_pre, d_post, d_bias, act, rows, n);
     return int(hipGetLastError());
 }
 
