@@ -7,12 +7,14 @@ import pytest
 
 import oracle
 import welvet_amd as wv
+from test_gpu_parity import shared_scale_blob
 
 pytestmark = pytest.mark.gpu
 
 TOL = 1e-5  # the f32 bar of wv_matvec, max |dy| / max |y| of each batch row
 FMTS = ["Q2_K", "Q3_K", "Q4_K", "Q5_K", "Q6_K", "Q8_0", "Q4_0", "Q4_1", "Q5_0", "Q5_1", "IQ1_S", "IQ2_XXS", "IQ2_XS",
         "IQ3_XXS", "IQ3_S", "IQ4_XS", "IQ4_NL", "TernaryPacked", "BinaryPacked", "AffinePacked"]
+GROUPS = ["affine32", "affine128", "affine256", "binary128"]  # the group widths that pack() does not make
 
 
 @pytest.fixture(scope="module", autouse=True)
@@ -23,8 +25,11 @@ def device():
 
 
 def make(fmt, rows, cols, seed):
-    rng = np.random.default_rng(seed)
-    p = wv.pack(fmt, (rng.standard_normal(rows * cols) * 0.02).astype(np.float32), rows, cols)
+    if fmt in GROUPS:
+        p, rng = shared_scale_blob(fmt, rows, cols, seed)
+    else:
+        rng = np.random.default_rng(seed)
+        p = wv.pack(fmt, (rng.standard_normal(rows * cols) * 0.02).astype(np.float32), rows, cols)
     return p, wv.upload(p), rng
 
 
@@ -37,8 +42,9 @@ def rowwise(y, ref):
     return float((np.abs(y - ref).max(1) / np.abs(ref).max(1)).max())
 
 
-@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("fmt", FMTS + GROUPS)
 def test_batched_forward_formats(fmt):
+    """Every format that the batched kernel takes; IQ4_NL, which it does not, runs on the one-row kernel."""
     rows, cols = 2000, 2304  # a ragged last row group; 9 super-blocks: waves of two, the last of one
     print(f"[gpu] batched {fmt}", flush=True)
     p, d, rng = make(fmt, rows, cols, 11)
@@ -222,7 +228,7 @@ def test_batches_under_capture_record_plain_launches(case):
     d.free()
 
 
-@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("fmt", FMTS + GROUPS)
 def test_batched_gradient_formats(fmt):
     rows, cols = 4700, 2304  # a ragged last row group; 9 super-blocks over the 8 XCDs; one slice of 8 waves
     print(f"[gpu] batched gradient {fmt}", flush=True)
@@ -243,7 +249,29 @@ def test_batched_gradient_tiles(shape):
     d.free()
 
 
-@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("fmt", ["Q4_K", "Q6_K", "Q8_0", "Q4_1", "IQ1_S"])
+def test_batched_gradient_nonfinite(fmt):
+    """NaN and infinities of gy reach every column of their own row, with the infinity's sign where they stay one, and
+    no other row's."""
+    rows, cols = 9001, 2304
+    print(f"[gpu] batched gradient non-finite {fmt}", flush=True)
+    p, d, rng = make(fmt, rows, cols, 23)
+    gy = rng.standard_normal((10, rows)).astype(np.float32)
+    gx = rng.standard_normal((10, cols)).astype(np.float32)
+    gy[1, 3], gy[2, 4000], gy[9, rows - 1] = np.nan, np.inf, -np.inf
+    w = oracle.unpack(oracle.Packed(p.fmt, p.rows, p.cols, p.raw, p.scales, p.meta, p.block_weights, p.mins))
+    w = w.reshape(rows, cols).astype(np.float64)
+    got = d.matvec_t(gy, gx)
+    assert np.isnan(got[1]).all()
+    for b, r in ((2, 4000), (9, rows - 1)):
+        inf = np.isinf(got[b])
+        assert (inf | np.isnan(got[b])).all() and (np.sign(got[b][inf]) == np.sign(gy[b, r] * w[r][inf])).all()
+    live = [0, 3, 4, 5, 6, 7, 8]
+    assert rowwise(got[live].astype(np.float64), gx[live] + gy[live].astype(np.float64) @ w) <= TOL
+    d.free()
+
+
+@pytest.mark.parametrize("fmt", FMTS + GROUPS)
 def test_batched_gradient_one_pass(fmt):
     """A shape whose batched plan fills the GPU once, which every format takes: 141 row groups over 8 waves, chains of
     18 with a ragged end, 9 super-blocks, quartets of rows and two left over."""

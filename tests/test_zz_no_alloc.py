@@ -1,7 +1,8 @@
 """wv_matvec_dev_noalloc (no device allocation, a fixed per-GPU scratch array)
 against wv_matvec_dev through the C ABI: calls in a row on K-split shapes,
-each smaller than the last, and batches past 8 rows (the K-split forward
-runs 8 rows per launch, so those launches reuse the array in stream order),
+each smaller than the last, and batches past 8 rows (the one-row kernels'
+K-split forward runs 8 rows per launch, so those launches reuse the array in
+stream order; the batched kernel's K split takes them in one),
 each bit-identical to the allocating entry point (same kernels and launch
 plan) and within 1e-5 normwise of the f64 oracle. Also: a shape whose
 partials exceed the array is refused before anything is enqueued, and a call
@@ -59,12 +60,12 @@ def test_noalloc_matches_allocating_entry_point():
         assert normwise(b, ref) <= 1e-5
 
 
-@pytest.mark.parametrize("batch", [9, 17])
-def test_noalloc_batches_past_one_split_launch(batch):
-    # 9 rows run as launches of 8 + 1, 17 as 8 + 8 + 1, all through the same
-    # partials in the array.
-    print(f"[gpu] no-alloc Q4_K 512x16384 batch {batch}", flush=True)
-    a, b, ref = run_pair("Q4_K", 512, 16384, batch, 77 + batch)
+@pytest.mark.parametrize("rows,batch", [(512, 9), (512, 17), (300, 17)])
+def test_noalloc_batches_past_one_split_launch(rows, batch):
+    # 9 rows run as launches of 8 + 1, 17 of 300 outputs as 8 + 8 + 1, all through the same
+    # partials in the array; 17 of 512 are work enough for the batched kernel, which splits K 16 ways.
+    print(f"[gpu] no-alloc Q4_K {rows}x16384 batch {batch}", flush=True)
+    a, b, ref = run_pair("Q4_K", rows, 16384, batch, 77 + batch)
     assert np.array_equal(a, b)
     assert normwise(b, ref) <= 1e-5
 
