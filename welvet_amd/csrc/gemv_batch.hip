@@ -19,16 +19,17 @@
 //     the one-row kernels' fixed point holds 2^-23 of a 32-column chunk's
 //     largest. Without the 2^12, lo's smallest step left 2^-39, and a dead
 //     channel of 1e8 beside N(0, 1) cost Q4_1 2.9e-5. hi and lo are different
-//     rows of the A operand, so one product gives both sums of 8 or 16 batch rows;
+//     rows of the A operand, so one product gives both sums of 8 or 16 batch rows.
+//     The 16-column sums of x that meet the k-quants' byte mins are such pairs
+//     of a 32nd of the sum, within 2^-46 of the largest x;
 //   * D holds exact products summed in f32; the group's scale meets it in f32
 //     FMAs on the VALU, 2^-s once per super-block.
-// Measured (Q4_K, us a call, one row kernel before): 4096->14336 12.9 / 15.1 /
-// 20.6 / 38 at 2 / 8 / 16 / 32 rows against 13.9 / 42.6 / 80 / 155;
-// 14336->4096 8 rows 17.4 against 67.4; Q8_0 4096->4096 32 rows 15.4 against
-// 62. 2-norm error against f64, 8 rows: 5.5e-7 through gate, up and down
+// Measured (Q4_K, us a call, one-row kernel before): 4096->14336 13.4 / 14.2 /
+// 19.9 at 2 / 8 / 16 rows against 13.8 / 37 / 72; 14336->4096 8 rows 16.7
+// against 65; Q8_0 4096->4096 32 rows 14.6 against 89. 2-norm error against f64, 8 rows: 5.5e-7 through gate, up and down
 // against 1.4e-6; Q8_0 1.1e-7 against 3.2e-7. What bounds it: at 8 rows the
 // weights would stream in 8 us; a wave's VALU work (about 630 instructions a
-// super-block for the operands and sums, 400 for converting 8 rows of x) and
+// super-block for the operands and sums, 450 for converting 8 rows of x) and
 // its load latencies at two waves per SIMD overlap only in part. 16 waves of
 // 128 registers spilled (24 us), and a form whose 8 waves share one
 // converted x, a chunk each, ran 19 us: its per-chunk metadata loads fill the
@@ -76,6 +77,8 @@ struct GemvBLds {
 constexpr int kBWaves = 8;  // per block at most: two of 256 registers on each SIMD
 
 constexpr uint32_t kInfBits = 0x7F800000u;
+constexpr uint32_t kLoBits = 12;  // lo halves are held at 2^12 times their place
+constexpr float kLoScale = float(1u << kLoBits);
 __device__ __forceinline__ uint32_t abs_bits(float f) { return __float_as_uint(f) & 0x7FFFFFFFu; }
 __device__ __forceinline__ uint32_t max4_bits(float4 v) {
     const uint32_t a = max(abs_bits(v.x), abs_bits(v.y)), b = max(abs_bits(v.z), abs_bits(v.w));
@@ -114,12 +117,32 @@ __device__ __forceinline__ bool scale_fields(const float4 (&v)[4], uint32_t (&f)
         wave_max4(m, w);
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) f[i] = min(253u, 268u - (w[i] >> 23));
+    for (int i = 0; i < 4; ++i) f[i] = min(254u - kLoBits, 268u - (w[i] >> 23));
     return odd;
 }
-// 2^12 (x - float(h)), exact where h is the fp16 nearest x, |x| <= 2^15: at most 2^15
-constexpr float kLoScale = 4096.0f;
-__device__ __forceinline__ float rest(float x, _Float16 h) { return fmaf(float(h), -1.0f, x) * kLoScale; }
+// The fp16 nearest 2^-12 x of a pair, and the remainders x - 2^12 h, exact (|x|
+// <= 2^27) until they too are rounded to fp16 (at most 2^15): an instruction a
+// half, 3 an element with the scaling. From float code the compiler takes 4.5
+// (the remainder's product, a conversion): 8 rows of Q4_K 4096->14336 14.9 us so
+// against 14.2, 16 rows of Q8_0 14336->4096 24.1 against 23.3.
+__device__ __forceinline__ uint32_t hi_pair(float a, float b) {
+    uint32_t h;
+    asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(h) : "v"(a), "s"(1.0f / kLoScale));
+    asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(h) : "v"(b), "s"(1.0f / kLoScale));
+    return h;
+}
+__device__ __forceinline__ uint32_t lo_pair(uint32_t h, float a, float b) {
+    uint32_t l;
+    asm("v_fma_mixlo_f16 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(l) : "v"(h), "s"(-kLoScale), "v"(a));
+    asm("v_fma_mixhi_f16 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(l) : "v"(h), "s"(-kLoScale), "v"(b));
+    return l;
+}
+__device__ __forceinline__ float rest(float x, _Float16 h) { return fmaf(float(h), -kLoScale, x); }
+// lo_pair with 0 for a remainder that is not finite (inf - inf)
+__device__ __forceinline__ uint32_t lo_pair_finite(uint32_t hb, float a, float b) {
+    const half2v h = __builtin_bit_cast(half2v, hb);
+    return pack_h2(finite_or_0(rest(a, h.x)), finite_or_0(rest(b, h.y)));
+}
 // The sum of a product's hi and lo rows.
 __device__ __forceinline__ float hi_lo(float hi, float lo) { return fmaf(lo, 1.0f / kLoScale, hi); }
 
@@ -190,49 +213,52 @@ __global__ void __launch_bounds__(64 * kBWaves) k_gemv_b(GemvBArgs ga) {
                 float sum[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const float up = __uint_as_float(f[i] << 23);
+                    const float up = __uint_as_float((f[i] + kLoBits) << 23);
                     v[i] = make_float4(v[i].x * up, v[i].y * up, v[i].z * up, v[i].w * up);
                     if constexpr (GP::kMin) sum[i] = (v[i].x + v[i].y) + (v[i].z + v[i].w);
                 }
-                // A non-finite x takes part as itself, in the code products and in the group sums, and
-                // leaves no output of its row finite. With f32 mins, whose group's products and sum may
-                // be infinities of opposite signs, it does so through the sum alone, as in the one-row kernels.
-                if (odd && kVM) {
+                uint2 h[4], d[4];  // columns 0 | 2 and 1 | 3
+                if (!odd) {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) v[i] = finite_or_0(v[i]);
+                    for (int i = 0; i < 4; ++i) {
+                        h[i] = make_uint2(hi_pair(v[i].x, v[i].z), hi_pair(v[i].y, v[i].w));
+                        d[i] = make_uint2(lo_pair(h[i].x, v[i].x, v[i].z), lo_pair(h[i].y, v[i].y, v[i].w));
+                    }
+                } else {
+                    // A non-finite x takes part as itself, in the code products and in the group sums, and
+                    // leaves no output of its row finite. With f32 mins, whose group's products and sum may
+                    // be infinities of opposite signs, it does so through the sum alone, as in the one-row kernels.
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float4 w = kVM ? finite_or_0(v[i]) : v[i];
+                        h[i] = make_uint2(hi_pair(w.x, w.z), hi_pair(w.y, w.w));
+                        d[i] = make_uint2(lo_pair_finite(h[i].x, w.x, w.z), lo_pair_finite(h[i].y, w.y, w.w));
+                    }
                 }
-                half2v h02[4], h13[4];
-                float4 d[4];
+                if constexpr (GP::kMin) {  // the group sums of x, in every lane of a group; four rows hide a DPP's wait
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) sum[i] += quad_xor1(sum[i]);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) sum[i] += quad_xor2(sum[i]);
+                    if constexpr (GW == 32) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) sum[i] += half_mirror(sum[i]);
+                    }
+                }
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    h02[i] = half2v{_Float16(v[i].x), _Float16(v[i].z)};
-                    h13[i] = half2v{_Float16(v[i].y), _Float16(v[i].w)};
-                    d[i] = make_float4(rest(v[i].x, h02[i].x), rest(v[i].y, h13[i].x), rest(v[i].z, h02[i].y),
-                                       rest(v[i].w, h13[i].y));
-                }
-                if (odd) {  // inf - inf
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) d[i] = finite_or_0(d[i]);
-                }
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    *reinterpret_cast<uint2*>(xw + (q + i) * 4) =
-                        make_uint2(__builtin_bit_cast(uint32_t, h02[i]), __builtin_bit_cast(uint32_t, h13[i]));
-                    *reinterpret_cast<uint2*>(xw + (NT + q + i) * 4) =
-                        make_uint2(pack_h2(d[i].x, d[i].z), pack_h2(d[i].y, d[i].w));
+                    *reinterpret_cast<uint2*>(xw + (q + i) * 4) = h[i];
+                    *reinterpret_cast<uint2*>(xw + (NT + q + i) * 4) = d[i];
                     xs[L::kInv + q + i] = __uint_as_float((254u - f[i]) << 23);
                     if constexpr (GP::kMin) {  // the lanes of a group store the same sum
                         float S = sum[i];
-                        S += quad_xor1(S);
-                        S += quad_xor2(S);
                         if constexpr (kMB) {
-                            S *= 0.03125f;  // at most 2^14
-                            const _Float16 h = _Float16(S);
-                            sw[(q + i) * 8] = h;
-                            sw[(NT + q + i) * 8] = _Float16(odd ? finite_or_0(rest(S, h)) : rest(S, h));
+                            S *= 0.03125f;  // at most 2^26
+                            const _Float16 sh = _Float16(S * (1.0f / kLoScale));
+                            sw[(q + i) * 8] = sh;
+                            sw[(NT + q + i) * 8] = _Float16(odd ? finite_or_0(rest(S, sh)) : rest(S, sh));
                         } else {
-                            if constexpr (GW == 32) S += half_mirror(S);
-                            xs[L::kSum + (lane / (GW / 4)) * NT + q + i] = S;
+                            xs[L::kSum + (lane / (GW / 4)) * NT + q + i] = S * (1.0f / kLoScale);
                         }
                     }
                 }
