@@ -1654,8 +1654,8 @@ __global__ void __launch_bounds__(1024) k_gemvt_rpl(RplArgs a, const float* __re
 // W * n row groups and NB rows; a weight's code is converted once and meets
 // the NB rows in an FMA each (205 VALU instructions per chunk and 4 rows, 64
 // per row there). 14336x4096 Q4_K, us: 3 / 8 / 16 rows 23.5 / 36.3 / 70 against
-// 32.3 / 57.9 / 111. VALU-bound: 22 us of 8 rows' 36 at one instruction per 4
-// cycles. Lane l ends with column l % 32 of rows 2s + l /
+// 32.3 / 57.9 / 111. VALU-bound: 26 us of 8 rows' 38 at one instruction per 4
+// cycles (15.8 M of them). Lane l ends with column l % 32 of rows 2s + l /
 // 32 for s = 0, 1. The lane sums are reduced after every 8 row groups: in one
 // chain of 28, 14336 rows came out 3.7e-7 from f64 against 2.9e-7, and as
 // slices of 64 row groups 8 rows took 47.5 us. Rows past the batch repeat its last one and go nowhere.
