@@ -293,7 +293,7 @@ def test_decoder_output_replaced_after_capture():
     dec.free()
 
 
-@pytest.mark.parametrize("rows,batch", [(7, 1), (1001, 1), (262144 - 256, 1), (262144 - 255, 1), (262144, 1), (300, 200), (300, 600)])
+@pytest.mark.parametrize("rows,batch", [(7, 1), (1001, 1), (262144 - 256 - 64, 1), (262144 - 256, 1), (262144 - 255, 1), (262144, 1), (300, 200), (300, 600)])
 def test_host_staging_sizes(rows, batch):
     """Host calls whose buffers fit the pinned bounce slot, end with it (256
     columns of x and these rows fill 1 MiB), pass it, and mix both (the input
